@@ -49,6 +49,8 @@ def _parse(lines):
 def _writes(op, ops):
     if not ops or op.startswith(_NO_VDST):
         return []
+    if op.startswith("buffer_load") and ops[-1].split()[-1] == "lds":
+        return []  # a direct-to-LDS load: its first operand is the address
     return _regs(ops[0])
 
 

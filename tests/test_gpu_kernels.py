@@ -460,6 +460,45 @@ def test_gemm_split_k_matches_oracle(torch, yuear_lib, oracle, m, n, k, residual
                                              None) == 1
 
 
+# tokens, features, K and epilogue that take each shape of the one-round form
+# on 256 CUs (gemm_ksplit_choice): ragged tiles in both directions, K of one
+# step (one wave has work), of fewer steps than waves, and of uneven shares
+@pytest.mark.parametrize("m,n,k,residual", [
+    (1, 100, 64, 0), (1, 99, 1600, 1), (49, 1028, 1600, 2), (66, 1027, 64, 1), (97, 2052, 576, 2),
+    (131, 1028, 1600, 0), (257, 1027, 576, 1), (200, 2050, 1600, 2), (97, 4100, 1600, 1),
+    (301, 3075, 576, 0), (131, 6150, 576, 2), (257, 4100, 192, 1), (301, 4099, 192, 0),
+    (513, 3076, 192, 1), (400, 4100, 576, 2), (700, 3075, 192, 0), (1010, 3070, 64, 2),
+    (700, 4100, 576, 1),
+])
+def test_gemm_few_tokens(torch, yuear_lib, oracle, m, n, k, residual):
+    """The K-split form of the GEMM (gemm_ksplit.hip) against the oracle on
+    padded rows: at most 64 rows compared, the padding of every row unchanged,
+    the same bits from a second launch."""
+    rng = np.random.default_rng(m + n + k)
+    lda, out_n = k + 8 * (m % 3), n // 2 if residual == 2 else n
+    ldc = out_n + m % 4
+    a = bf(rng.normal(size=(m, lda)))
+    w = bf(rng.normal(size=(n, k)) * 0.05)
+    c0 = bf(rng.normal(size=(m, ldc)))
+    da, dw = dev(torch, a), dev(torch, w)
+    outs = []
+    for _ in range(2):
+        dc = dev(torch, c0)
+        assert yuear_lib.lib.yuear_op_gemm(da.data_ptr(), lda, dw.data_ptr(), m, n, k,
+                                           dc.data_ptr(), ldc, residual, None) == 0
+        outs.append(host(torch, dc))
+    np.testing.assert_array_equal(outs[0], outs[1])
+    np.testing.assert_array_equal(outs[0][:, out_n:], c0[:, out_n:])
+    rows = np.unique(np.r_[0, m - 1, rng.integers(0, m, 62)])
+    acc = oracle.linear(np.ascontiguousarray(a[rows, :k]), w)
+    if residual == 2:
+        ref = oracle.silu_mul(acc[:, 0::2], acc[:, 1::2])
+    else:
+        ref = bf(f(c0[rows][:, :out_n]) + f(acc)) if residual else acc
+    scale = max(np.abs(f(acc)).max(), np.abs(f(ref)).max())
+    assert_close_bf16(outs[0][rows][:, :out_n], ref, scale=scale, exact_frac=0.9)
+
+
 @pytest.mark.parametrize("m,n,k", [(7, 1024, 3072), (3000, 3072, 8192), (700, 5120, 3072)])
 def test_gemm_split_k_is_deterministic(torch, yuear_lib, m, n, k):
     """Every output sums its K products in the same order on each launch (no

@@ -16,7 +16,8 @@ CSRC = os.path.join(ROOT, "yue2-mlx_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang",
          "-target-feature", "-Xclang", "-packed-fp32-ops", "--offload-device-only", "-S"]
-SOURCES = ["attention.hip", "prefill.hip", "nar_attention.hip", "gemm.hip", "gemv_mfma.hip"]
+SOURCES = ["attention.hip", "prefill.hip", "nar_attention.hip", "gemm.hip", "gemv_mfma.hip",
+           "gemm_ksplit.hip"]
 
 CLEAN = """_Zk:
 	global_load_dwordx4 v[2:5], v[10:11], off

@@ -29,7 +29,8 @@
 // the 256 x 256 tile were conflict stalls). Fragment of a 16-wide K sub-step
 // s: lane l reads row l % 32, chunk 2 s + l / 32.
 //
-// Tile shapes (launch_gemm picks the one with the least estimated time for
+// Tile shapes (past the sizes that gemm_ksplit.hip does in one round of
+// smaller tiles, launch_gemm picks the one with the least estimated time for
 // the shape and the CU count): 256 x 256 (8 waves of 128 x 64), 256 x 128 and
 // 128 x 256 (8 waves of 64 x 64), 256 x 192 (8 waves of 64 x 96), 192 x 192
 // (8 waves of 96 x 48) and 128 x 128 (4 waves of 64 x 64, two workgroups per
@@ -42,6 +43,7 @@
 #include <mutex>
 
 #include "common.h"
+#include "gemm_epilogue.h"
 #include "kernels.h"
 
 namespace yuear {
@@ -65,32 +67,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void *base, si
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0,
                                            uint32_t(bytes > 0xffffffffu ? 0xffffffffu : bytes),
                                            0x00020000);
-}
-
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  return uint32_t(f2bf(a)) | uint32_t(f2bf(b)) << 16;
-}
-
-// SwiGLU epilogue (ar.cpp:36-51) on interleaved (gate_i, up_i) columns: the
-// lane's features n .. n + 3 (n a multiple of 4) are two pairs, written as
-// outputs n / 2 and n / 2 + 1 of the row with the rounding points of the
-// decode GEMV's epilogue: g, u rounded to bf16, silu(g) rounded, then g * u.
-__device__ __forceinline__ uint16_t swiglu_one(float gate, float up) {
-  const float g = rbf(gate), u = rbf(up);
-  const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
-  return f2bf(act * u);
-}
-__device__ __forceinline__ void swiglu_store(const GemmParams &p, int m, int n, const float *v) {
-  uint16_t *c = p.c + size_t(m) * p.ldc + (n >> 1);
-  if (n + 3 < p.n && (p.ldc & 1) == 0) {
-    *reinterpret_cast<uint32_t *>(c) =
-        uint32_t(swiglu_one(v[0], v[1])) | uint32_t(swiglu_one(v[2], v[3])) << 16;
-  } else {
-    if (n + 1 < p.n)
-      c[0] = swiglu_one(v[0], v[1]);
-    if (n + 3 < p.n)
-      c[1] = swiglu_one(v[2], v[3]);
-  }
 }
 
 // silu(g) rounded to bf16 for every bf16 value g (index = g's bits), by the
@@ -122,34 +98,6 @@ __device__ __forceinline__ void swiglu_store_tab(const GemmParams &p, const uint
       c[0] = swiglu_tab(tab, v[0], v[1]);
     if (n + 3 < p.n)
       c[1] = swiglu_tab(tab, v[2], v[3]);
-  }
-}
-
-// Epilogue of a lane's 4 consecutive features n .. n + 3 (n a multiple of 4)
-// of token row m < p.m: the 8-byte form when all four are in range and rows
-// stay 8-byte aligned, else element by element.
-__device__ __forceinline__ void epilogue4(const GemmParams &p, int m, int n, const float *v) {
-  if (p.residual == 2) {
-    swiglu_store(p, m, n, v);
-    return;
-  }
-  uint16_t *c = p.c + size_t(m) * p.ldc + n;
-  if (n + 3 < p.n && (p.ldc & 3) == 0) {
-    uint2 o;
-    if (p.residual) {
-      const uint2 old = *reinterpret_cast<const uint2 *>(c);
-      o.x = pack_bf16x2(bf2f(uint16_t(old.x)) + rbf(v[0]), bf2f(uint16_t(old.x >> 16)) + rbf(v[1]));
-      o.y = pack_bf16x2(bf2f(uint16_t(old.y)) + rbf(v[2]), bf2f(uint16_t(old.y >> 16)) + rbf(v[3]));
-    } else {
-      o.x = pack_bf16x2(v[0], v[1]);
-      o.y = pack_bf16x2(v[2], v[3]);
-    }
-    *reinterpret_cast<uint2 *>(c) = o;
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (n + e < p.n)
-        c[e] = p.residual ? f2bf(bf2f(c[e]) + rbf(v[e])) : f2bf(v[e]);
   }
 }
 
@@ -804,6 +752,11 @@ int gemm_cus() { return device_cus(); }
 
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s) {
   const int cus = device_cus();
+  if (p.m > 0 && p.n > 0 && p.k >= kBK) {
+    const int few = gemm_ksplit_choice(p.m, p.n, p.k, cus);
+    if (few >= 0)
+      return launch_gemm_ksplit(p, few, s);
+  }
   int shape = gemm_tile_choice(p.m, p.n, cus), splits = 1;
   if (p.part)
     gemm_plan(p.m, p.n, p.k, cus, p.part_bytes, &shape, &splits);

@@ -195,6 +195,11 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s);
 // its split count.
 hipError_t launch_gemm_tile(const GemmParams &p, int shape, hipStream_t s, int splits = 1);
 int gemm_tile_choice(int m, int n, int cus);
+// The K-split form (gemm_ksplit.hip) for GEMMs that fit one round of its
+// tiles: the shape to launch, or -1 when there is none. launch_gemm takes it
+// first. No workspace; the sums' order depends on k and the shape only.
+int gemm_ksplit_choice(int m, int n, int k, int cus);
+hipError_t launch_gemm_ksplit(const GemmParams &p, int shape, hipStream_t s);
 int gemm_cus();  // CUs of the current device (256 if it cannot be read)
 // The reduce of a residual GEMM launched with defer_reduce and splits > 1
 // (c = bf16(c + bf16(sum of the splits in split order)), as
