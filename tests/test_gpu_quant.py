@@ -108,6 +108,19 @@ def test_qgemv_matches_oracle(torch, yuear_lib, oracle, bits, n, k, batch, norm,
     assert_close_bf16(got, ref, scale=scale, exact_frac=0.9)
 
 
+# the edges of the row-set rule (launch_lp): a last set of one row, one set
+# more than the workgroups, a third loop round, one row past a one-pass form,
+# rows of 6 and 8 pieces per lane
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("n,k,batch,epilogue", [
+    (4097, 3072, 2, 0), (4097, 3072, 1, 1), (16385, 3072, 2, 0), (16386, 3072, 1, 2),
+    (32770, 3072, 2, 2), (16385, 2048, 2, 1), (4097, 2048, 1, 0), (8193, 2048, 2, 0),
+    (602, 8192, 2, 2), (4099, 6144, 1, 0), (8193, 4096, 2, 0), (20000, 256, 2, 0),
+])
+def test_qgemv_row_sets(torch, yuear_lib, oracle, bits, n, k, batch, epilogue):
+    test_qgemv_matches_oracle(torch, yuear_lib, oracle, bits, n, k, batch, True, epilogue)
+
+
 def test_qgemv_rejects_unsupported_shapes(torch, yuear_lib):
     d = dev(torch, np.zeros(4096, np.uint32))
     y = dev(torch, np.zeros(64, np.uint16))

@@ -14,8 +14,9 @@
 // Streaming: a row is NP = k * bits / 128 16-byte pieces (32 codes at 4 bits,
 // 16 at 8). L lanes share a row (64 / L rows per wave), lane li reading the P
 // pieces li + p L, so each wave-wide load covers whole 16-byte pieces of
-// 64 / L rows; a wave owns R such row sets and issues all its loads (codes
-// non-temporal, group words with them) before the first use. The activation
+// 64 / L rows; a wave owns R such row sets (one pass, or in a loop over sets)
+// and issues all loads of a pass (codes non-temporal, group words with them)
+// before the first use. The activation
 // rows, gathered and RMS-normalised exactly as in the bf16 GEMV, are staged
 // once per workgroup in LDS, permuted so that every code pair meets its
 // activation pair, together with each piece's activation sum.
@@ -80,7 +81,7 @@ __device__ __forceinline__ u32x4 pair_order(u32x4 v) {
                  __builtin_amdgcn_perm(d, c, 0x05040100u), __builtin_amdgcn_perm(d, c, 0x07060302u)};
 }
 
-template <int B, int BITS, int L, int P, int R>
+template <int B, int BITS, int L, int P, int R, bool LOOP>
 __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
   constexpr int EP = 128 / BITS;          // codes per 16-byte piece
   constexpr int RW = 64 / L;              // rows per wave and row set
@@ -91,7 +92,11 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
   constexpr int XPT = (NCH + 255) / 256;  // chunks per thread when staging
   constexpr int CPP = EP / 8;             // chunks per piece (4 or 2)
   constexpr int GPR = K / 64;             // groups per row
-  __shared__ u32x4 xs[B][NCH];
+  // chunk j of piece q at j XS + q: the lanes of a wave, on consecutive
+  // pieces, read consecutive 16-byte slots (chunk order, CPP slots apart, left
+  // their reads CPP-way bank-conflicted); the padding spreads the writes
+  constexpr int XS = NP + (CPP == 4 ? 4 : 8);
+  __shared__ u32x4 xs[B][CPP * XS];
   __shared__ float psum[B][NP];
   __shared__ float red[B][4];
   __shared__ float res[B][ROWS];
@@ -117,22 +122,26 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
       gr[i] = reinterpret_cast<const u32x4 *>(p.norm_w)[min(tid + 256 * i, NCH - 1)];
   }
 
-  // 2. Code and group-word stream of this wave's rows.
-  u32x4 wv[R][P];
-  uint32_t sbv[R][P];
+  // 2. Code and group-word stream of this wave's rows of row set `set` (past
+  // the last set: its last rows again, never used).
+  u32x4 wv[LOOP ? 2 : 1][R][P];
+  uint32_t sbv[LOOP ? 2 : 1][R][P];
+  auto load = [&](int buf, int set) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int lr = min(blk * ROWS + (wave * R + r) * RW + sub, p.n - 1);
-    const int row = lr < p.seg0_len ? p.seg0_start + lr : p.seg1_start + (lr - p.seg0_len);
-    const u32x4 *wrow = reinterpret_cast<const u32x4 *>(p.qw) + size_t(row) * NP;
-    const uint32_t *srow = p.qsb + size_t(row) * GPR;
+    for (int r = 0; r < R; ++r) {
+      const int lr = min(set * ROWS + (wave * R + r) * RW + sub, p.n - 1);
+      const int row = lr < p.seg0_len ? p.seg0_start + lr : p.seg1_start + (lr - p.seg0_len);
+      const u32x4 *wrow = reinterpret_cast<const u32x4 *>(p.qw) + size_t(row) * NP;
+      const uint32_t *srow = p.qsb + size_t(row) * GPR;
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
-      const int piece = li + q * L;
-      wv[r][q] = __builtin_nontemporal_load(wrow + piece);
-      sbv[r][q] = __builtin_nontemporal_load(srow + piece / (64 / EP));
+      for (int q = 0; q < P; ++q) {
+        const int piece = li + q * L;
+        wv[buf][r][q] = __builtin_nontemporal_load(wrow + piece);
+        sbv[buf][r][q] = __builtin_nontemporal_load(srow + piece / (64 / EP));
+      }
     }
-  }
+  };
+  load(0, blk);
 
   // 3. Stage: RMSNorm (the bf16 GEMV's arithmetic and order), the gathered
   // rows to x_out, piece sums, pair order.
@@ -199,7 +208,7 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
       if constexpr (CPP == 4)
         cs += dpp<0x4E>(cs);
       if (c < NCH) {
-        xs[b][c] = pair_order<BITS>(v);
+        xs[b][(c % CPP) * XS + c / CPP] = pair_order<BITS>(v);
         if (c % CPP == 0)
           psum[b][c / CPP] = cs;
       }
@@ -207,104 +216,124 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
   }
   __syncthreads();
 
-  // 4. Dot products.
-  float acc[R][B];
+  // 4. Row set blk, or with LOOP blk, blk + gridDim.x, ...: the next set's
+  // loads are issued before this one's products, and no barrier separates the
+  // sets (a wave's sums pass through its own part of `res`).
+  float *own = &res[0][0] + wave * (R * RW * B);  // [B][R * RW]
+  auto products = [&](int buf, int set) {
+    float acc[R][B];
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int b = 0; b < B; ++b)
-      acc[r][b] = 0.f;
+      for (int b = 0; b < B; ++b)
+        acc[r][b] = 0.f;
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    const int piece = li + q * L;
-    uint32_t xw[B][CPP * 4];
-    float sx[B];
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-#pragma unroll
-      for (int j = 0; j < CPP; ++j) {
-        const u32x4 v = xs[b][piece * CPP + j];
-        xw[b][4 * j] = v.x;
-        xw[b][4 * j + 1] = v.y;
-        xw[b][4 * j + 2] = v.z;
-        xw[b][4 * j + 3] = v.w;
-      }
-      sx[b] = psum[b][piece];
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const u32x4 w = wv[r][q];
-      const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
-      uint32_t pr[4][4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-          pr[j][s] = ((wd[j] >> (4 * s)) & kPairMask) | kPairBias;
-      const float sc = bflo(sbv[r][q]), bias = bfhi(sbv[r][q]);
+    for (int q = 0; q < P; ++q) {
+      const int piece = li + q * L;
+      uint32_t xw[B][CPP * 4];
+      float sx[B];
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        if constexpr (BITS == 4) {
-          float d0 = 0.f, d1 = 0.f;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {  // word j <-> chunk j
-            d0 = dot2(pr[j][0], xw[b][4 * j], d0);
-            d1 = dot2(pr[j][1], xw[b][4 * j + 1], d1);
-            d0 = dot2(pr[j][2], xw[b][4 * j + 2], d0);
-            d1 = dot2(pr[j][3], xw[b][4 * j + 3], d1);
-          }
-          const float cb = __builtin_fmaf(-128.f, sc, bias);
-          acc[r][b] = __builtin_fmaf(sc, d0 + d1, __builtin_fmaf(cb, sx[b], acc[r][b]));
-        } else {
-          float lo = 0.f, hi = 0.f;
+        for (int j = 0; j < CPP; ++j) {
+          const u32x4 v = xs[b][j * XS + piece];
+          xw[b][4 * j] = v.x;
+          xw[b][4 * j + 1] = v.y;
+          xw[b][4 * j + 2] = v.z;
+          xw[b][4 * j + 3] = v.w;
+        }
+        sx[b] = psum[b][piece];
+      }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {  // word j: elements 4j..4j+3, pairs (0,2), (1,3)
-            const uint32_t x02 = xw[b][2 * j], x13 = xw[b][2 * j + 1];
-            lo = dot2(pr[j][0], x02, lo);
-            hi = dot2(pr[j][1], x02, hi);
-            lo = dot2(pr[j][2], x13, lo);
-            hi = dot2(pr[j][3], x13, hi);
+      for (int r = 0; r < R; ++r) {
+        const u32x4 w = wv[buf][r][q];
+        const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+        uint32_t pr[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            pr[j][s] = ((wd[j] >> (4 * s)) & kPairMask) | kPairBias;
+        const float sc = bflo(sbv[buf][r][q]), bias = bfhi(sbv[buf][r][q]);
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          if constexpr (BITS == 4) {
+            float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {  // word j <-> chunk j
+              d0 = dot2(pr[j][0], xw[b][4 * j], d0);
+              d1 = dot2(pr[j][1], xw[b][4 * j + 1], d1);
+              d0 = dot2(pr[j][2], xw[b][4 * j + 2], d0);
+              d1 = dot2(pr[j][3], xw[b][4 * j + 3], d1);
+            }
+            const float cb = __builtin_fmaf(-128.f, sc, bias);
+            acc[r][b] = __builtin_fmaf(sc, d0 + d1, __builtin_fmaf(cb, sx[b], acc[r][b]));
+          } else {
+            float lo = 0.f, hi = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {  // word j: elements 4j..4j+3, pairs (0,2), (1,3)
+              const uint32_t x02 = xw[b][2 * j], x13 = xw[b][2 * j + 1];
+              lo = dot2(pr[j][0], x02, lo);
+              hi = dot2(pr[j][1], x02, hi);
+              lo = dot2(pr[j][2], x13, lo);
+              hi = dot2(pr[j][3], x13, hi);
+            }
+            const float cb = __builtin_fmaf(-2176.f, sc, bias);
+            acc[r][b] = __builtin_fmaf(sc, __builtin_fmaf(16.f, hi, lo),
+                                       __builtin_fmaf(cb, sx[b], acc[r][b]));
           }
-          const float cb = __builtin_fmaf(-2176.f, sc, bias);
-          acc[r][b] = __builtin_fmaf(sc, __builtin_fmaf(16.f, hi, lo),
-                                     __builtin_fmaf(cb, sx[b], acc[r][b]));
         }
       }
     }
-  }
 
-  // 5. Row sums, then the epilogue over the workgroup's rows.
+    // 5. Row sums, then the epilogue of the wave's rows, one lane per (row or
+    // pair, branch).
+    __builtin_amdgcn_wave_barrier();  // the last set's sums have been read
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const float t = group_sum<L>(acc[r][b]);
-      if (li == 0)
-        res[b][(wave * R + r) * RW + sub] = t;
-    }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-    uint16_t *yb = p.y + size_t(b) * p.y_stride;
+      for (int b = 0; b < B; ++b) {
+        const float t = group_sum<L>(acc[r][b]);
+        if (li == 0)
+          own[b * (R * RW) + r * RW + sub] = t;
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int row0 = set * ROWS + wave * (R * RW);
     if (p.epilogue == kEpiSwiGLU) {
-      for (int i = tid; i < ROWS / 2; i += 256) {
-        const int row = blk * ROWS + 2 * i;
-        if (row + 1 < p.n) {
-          const float g = rbf(res[b][2 * i]), u = rbf(res[b][2 * i + 1]);
+      if constexpr (R * RW % 2 == 0) {
+        const int b = lane / (R * RW / 2), i = lane % (R * RW / 2), row = row0 + 2 * i;
+        if (b < B && row + 1 < p.n) {
+          const float g = rbf(own[b * (R * RW) + 2 * i]), u = rbf(own[b * (R * RW) + 2 * i + 1]);
           const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
-          yb[row >> 1] = f2bf(act * u);
+          p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
         }
       }
     } else {
-      for (int i = tid; i < ROWS; i += 256) {
-        const int row = blk * ROWS + i;
-        if (row < p.n) {
-          float v = res[b][i];
-          if (p.epilogue == kEpiResidual)
-            v = bf2f(yb[row]) + rbf(v);
-          yb[row] = f2bf(v);
-        }
+      const int b = lane / (R * RW), i = lane % (R * RW), row = row0 + i;
+      if (b < B && row < p.n) {
+        uint16_t *y = p.y + size_t(b) * p.y_stride + row;
+        float v = own[b * (R * RW) + i];
+        if (p.epilogue == kEpiResidual)
+          v = bf2f(*y) + rbf(v);
+        *y = f2bf(v);
       }
+    }
+  };
+  if constexpr (!LOOP) {
+    products(0, blk);
+  } else {
+    const int step = int(gridDim.x), sets = (p.n + ROWS - 1) / ROWS;
+    for (int set = blk; set < sets; set += 2 * step) {
+      const bool more = set + step < sets;  // uniform
+      if (more)
+        load(1, set + step);
+      products(0, set);
+      if (!more)
+        break;
+      if (set + 2 * step < sets)
+        load(0, set + 2 * step);
+      products(1, set + step);
     }
   }
   if (p.advance && blk == 0 && tid < p.batch)
@@ -330,31 +359,61 @@ bool qgemv_shape(int bits, int k, Shape &s) {
   return false;
 }
 
-template <int B, int BITS, int L, int P, int R>
-hipError_t launch_r(const GemvParams &p, hipStream_t s) {
-  constexpr int rows = 4 * R * (64 / L);
-  hipLaunchKernelGGL((qgemv_kernel<B, BITS, L, P, R>), dim3((p.n + rows - 1) / rows), dim3(256),
-                     0, s, p);
+template <int B, int BITS, int L, int P, int R, bool LOOP>
+hipError_t launch_r(const GemvParams &p, hipStream_t s, int grid) {
+  hipLaunchKernelGGL((qgemv_kernel<B, BITS, L, P, R, LOOP>), dim3(grid), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
+// Row sets per wave (R) and per workgroup. The RMSNorm prologue, which every
+// workgroup repeats, is ~500 VALU instructions a wave at batch 2 (as many as
+// the products of 16 rows), so a normed launch takes fewer workgroups that
+// loop over row sets with the next set's loads in flight: 512 of them, two
+// per CU, or 1024 where a row is one or two pieces per lane and the registers
+// allow. At batch 1 or for short rows, one pass of four sets is the faster
+// form while it leaves 512-1024 workgroups (short rows at batch 1: always,
+// 32769 x 2048 9.6 against 9.9 us looped). Measured on MI355X, us, cold
+// weights, before (one pass, at least 1024 workgroups) -> now, batch 1 / 2:
+//   4 bits: 5120 x 3072  5.1 -> 4.6 / 7.6 -> 6.0;  16384 x 3072 SwiGLU
+//   8.4 -> 8.5 / 12.6 -> 10.2;  83968 x 3072  26.8 -> 26.3 / 41.0 -> 32.2;
+//   12288 x 2048 SwiGLU  5.9 -> 5.5 / 8.3 -> 7.0
+//   8 bits: 6.8 -> 6.0 / 9.5 -> 7.6;  13.2 -> 12.8 / 16.7 -> 16.0;
+//   47.6 -> 46.4 / 65.2 -> 57.4;  7.8 -> 7.7 / 10.6 -> 9.6
+// Without a norm the staging is cheap and more workgroups win (3072 x 8192 at
+// 8 bits, batch 2: 10.3 in one pass, 12.2 in the loop).
 template <int B, int BITS, int L, int P>
 hipError_t launch_lp(const GemvParams &p, hipStream_t s) {
-  // more row sets per wave for the long GEMVs (lm_head, gate/up) while that
-  // still leaves >= 1024 workgroups: each workgroup's activation staging is
-  // then shared by more rows (4-bit lm_head: 47.7 / 36.1 / 31.9 us with
-  // 1 / 2 / 4 sets); one set for the short ones, whose time is latency
+  auto sets = [&](int r) { return (p.n + 4 * r * (64 / L) - 1) / (4 * r * (64 / L)); };
+  constexpr bool kShort = P <= 2;
   if constexpr (P <= 3) {
-    constexpr int rows4 = 16 * (64 / L);
-    if ((p.n + rows4 - 1) / rows4 >= 1024)
-      return launch_r<B, BITS, L, P, 4>(p, s);
+    if (p.norm_w) {
+      if constexpr (B == 1 || kShort) {
+        if (sets(4) >= 512 && ((B == 1 && kShort) || sets(4) <= 1024))
+          return launch_r<B, BITS, L, P, 4, false>(p, s, sets(4));
+      }
+      if (sets(2) >= 1024)
+        return launch_r<B, BITS, L, P, 2, true>(p, s, kShort ? 1024 : 512);
+      if constexpr (kShort) {
+        if (sets(2) >= 512)
+          return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
+      }
+      if (sets(1) > 512 && (L < 64 || p.epilogue != kEpiSwiGLU))
+        return launch_r<B, BITS, L, P, 1, true>(p, s, 512);
+    }
+  }
+  if constexpr (P <= 3) {
+    if (sets(4) >= 1024)
+      return launch_r<B, BITS, L, P, 4, false>(p, s, sets(4));
   }
   if constexpr (P <= 4) {
-    constexpr int rows2 = 8 * (64 / L);
-    if ((p.n + rows2 - 1) / rows2 >= 1024)
-      return launch_r<B, BITS, L, P, 2>(p, s);
+    if (sets(2) >= 1024)
+      return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
   }
-  return launch_r<B, BITS, L, P, 1>(p, s);
+  if constexpr (L == 64) {  // a (gate, up) pair stays in one wave
+    if (p.epilogue == kEpiSwiGLU)
+      return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
+  }
+  return launch_r<B, BITS, L, P, 1, false>(p, s, sets(1));
 }
 
 template <int B, int BITS>
