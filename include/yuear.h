@@ -344,10 +344,12 @@ int32_t yuear_op_attention_prefill(const uint16_t *dev_q,
  * otherwise, nar_attention.cpp:245-268). This entry point computes those
  * with the same precise kernel too: their parity with the reference is
  * unpinned. workspace: yuear_nar_attention_workspace_bytes()
- * of device memory. A non-causal launch too small to fill the GPU splits
- * its keys over workgroups; the split partials come from a library pool
- * per (device, stream). So the first such call on a stream, or one that
- * needs a larger pool, allocates: make it outside graph capture. Runs on
+ * of device memory (required; the kernels of this version read V as given and
+ * leave it untouched). Non-causal launches may deal the keys of a query tile
+ * to several workgroups; their partials (at most 35 MB) come from a library
+ * pool per (device, stream). So the first such call on a stream, or one that
+ * needs a larger pool, allocates: make it outside graph capture, where such a
+ * call runs undealt (slower; sums in another order). Runs on
  * `stream` (a hipStream_t, NULL = default); the reference's ValueError
  * messages for invalid shapes. */
 int64_t yuear_nar_attention_workspace_bytes(int32_t batch, int32_t kv_heads, int32_t kv_len);

@@ -58,6 +58,8 @@ def _origin(insts, idx, reg):
     j = idx - 1
     while j >= 0:
         op, ops = insts[j]
+        if op.startswith("v_mfma") and reg in _regs(ops[0]):
+            return ("valu", j)  # a score, from which the P pieces are made
         if reg in _writes(op, ops):
             if op.startswith(_LOADS):
                 return ("load", j)
@@ -97,6 +99,11 @@ def check_function(lines):
             origins = [_origin(insts, idx, r) for r in regs]
             kinds = {o[0] for o in origins}
             loads = {o[1] for o in origins if o[0] == "load"}
+            # two transposing LDS reads build a tuple, one half each
+            if (kinds == {"load"} and len(loads) == 2 and len(regs) == 4 and
+                    all(insts[j][0].startswith("ds_read_b64_tr") for j in loads) and
+                    origins[0] == origins[1] and origins[2] == origins[3]):
+                continue
             if ("load" in kinds and len(kinds) > 1) or len(loads) > 1:
                 bad.append((op + " " + ", ".join(ops),
                             [(k, " ".join([insts[j][0]] + insts[j][1]) if j >= 0 else "")

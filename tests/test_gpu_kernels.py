@@ -604,3 +604,14 @@ def test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, hea
         assert yuear_lib.lib.yuear_op_attention_prefill(
             a[0].data_ptr(), a[1].data_ptr(), a[2].data_ptr(), t_, p0, hq, kv_heads, cap,
             out.data_ptr(), None) == 1, (t_, p0, hq)
+
+
+@pytest.mark.parametrize("T,pos0,heads,kv_heads", [
+    # key-split tiles of 16 queries by 4 and by 8 waves: one block, one block a
+    # wave and one more, a last query tile of one; of 32 queries by 8 and by 4;
+    # 64-query tiles with an odd last block (tail step) and a ragged last tile
+    (1, 0, 1, 1), (16, 240, 8, 8), (17, 240, 6, 2), (160, 97, 24, 8), (33, 2000, 24, 8),
+    (301, 607, 24, 8), (341, 0, 24, 8), (700, 0, 24, 8), (681, 1969, 24, 8),
+])
+def test_attention_prefill_tile_forms(torch, yuear_lib, oracle, T, pos0, heads, kv_heads):
+    test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, heads, kv_heads)

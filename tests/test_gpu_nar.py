@@ -63,6 +63,23 @@ def test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, 
     assert_close_bf16(host(torch, got), ref, exact_frac=0.8)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk,causal", [
+    # whole key-split tiles of 16 and 32 queries, 4 and 8 waves: fewer blocks
+    # than waves, a partial last block, a last tile of one query
+    (1, 1, 1, 1, 31, False), (2, 6, 3, 17, 289, False), (1, 1, 1, 1, 697, False),
+    (1, 24, 8, 651, 31, False), (1, 6, 3, 677, 919, False),
+    # dealt: 9, 9, 8 and 13 pieces a tile at most, a ragged last tile, steps
+    # and blocks that do not divide
+    (2, 16, 8, 1, 4001, False), (1, 16, 8, 53, 2000, False), (1, 24, 8, 53, 6500, False),
+    (1, 6, 3, 274, 6000, False), (1, 16, 8, 100, 8001, False), (1, 24, 8, 250, 3600, False),
+    # 64-query tiles, an odd last block; causal forms
+    (1, 12, 4, 677, 31, False), (1, 24, 8, 1024, 400, False), (1, 24, 8, 100, 100, True),
+    (1, 24, 8, 449, 449, True), (1, 48, 16, 850, 850, True),
+])
+def test_nar_attention_tile_forms(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal):
+    test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal)
+
+
 def test_nar_attention_zero_pads_the_last_key_block(torch, yuear_lib, oracle):
     # 50 keys leave 14 padding slots in the last 32-key block of the
     # workspace: a workspace full of NaN must not reach the output

@@ -1,24 +1,22 @@
-// One 32-query tile of multi-query attention with head_dim 128 on gfx950
-// MFMA, shared by the causal prefill attention (prefill.hip, ar.cpp:284-291)
-// and the acoustic-model attention (nar_attention.hip,
-// nar_attention.cpp:63-218): fp32 scores of bf16 operands, an exp2 online
-// softmax in fp32, P fed to P.V as three truncated bf16 pieces (its 24
-// significant bits: every product exact), fp32 sums, bf16(o / l).
-//
-// The workgroup's 4 waves split the tile's key range: wave w walks the
-// 32-key blocks w, w + 4, w + 8, ... with the next block's K loads in flight
-// (and the block's own V issued at its start), then the four (m, l, O)
-// partials are merged through LDS. Each wave holds both 16-query MFMA column
-// tiles:
+// Query tiles of multi-query attention with head_dim 128 on gfx950 MFMA,
+// shared by the causal prefill attention (prefill.hip, ar.cpp:284-291) and
+// the acoustic-model attention (nar_attention.hip, nar_attention.cpp:63-218):
+// fp32 scores of bf16 operands, an exp2 online softmax in fp32, P fed to P.V
+// as three truncated bf16 pieces (its 24 significant bits: every product
+// exact), fp32 sums, bf16(o / l).
 //
 //   S^T[key][query] = K[key][:] . q[query][:]            (attn_core.h rows)
 //   O^T[dim][query] += V^T[dim][key] . P^T[key][query]
 //
-// Splitting the keys over the waves (rather than the queries) shortens each
-// wave's dependent chain of blocks four times and gives four times more
-// workgroups; both matter because a block step is a latency-bound chain
-// (MFMA accumulations, cross-lane max / sum, the exp2 and the P split).
+// Two forms. The key-split tile (attn_query_tile, 16 or 32 queries) has its 4
+// or 8 waves split the tile's 32-key blocks and merges their (m, l, O) through
+// LDS: for launches with few tiles, whose time is the longest wave's chain of
+// blocks and the rate at which one CU pulls K and V (4 waves: two workgroups
+// to a CU, for more tiles than CUs). The 64-query tile
+// (attn_query_tile64) has its 4 waves walk the same blocks, fetched once per
+// workgroup: for launches that fill the GPU, bound by VALU and MFMA issue.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_core.h"
@@ -27,135 +25,259 @@
 namespace yuear {
 namespace attn {
 
-struct TileLds {
-  float m[4][2][16], l[4][2][16];
-  f32x4 o[4][2][8][64];  // [wave][column tile][dim tile][lane]
-};
-
 struct QueryTile {
   const u32x4 *kc = nullptr;  // this kv head's K rows, row-major [slot][128]
-  const u32x4 *vc = nullptr;  // its V in 32-key dim-major blocks (v_index)
+  const u32x4 *vc = nullptr;  // its V in 32-key dim-major blocks (v_index) or as rows
   int kend = 0;               // keys [0, kend) are read
   int kv_len = 0;             // non-causal: keys [0, kv_len) are visible
   int causal_pos = -1;        // >= 0: query t sees keys <= causal_pos + t
   const uint16_t *q = nullptr;  // query 0 of the tile
   size_t q_stride = 0;          // elements between consecutive queries
-  int nq = 0;                   // valid queries (1..32)
+  int nq = 0;                   // valid queries of the tile
   uint16_t *out = nullptr;      // output row of query 0
   size_t out_stride = 0;
-  // attn_query_tile64 only: key blocks [blk0, blk1) of the tile (blk1 0: all)
-  // and, when set, an unnormalised partial per query instead of out: 132
+  // key-split tile, non-causal: key blocks [blk0, blk1) of the tile (blk1 0:
+  // all) and, when set, an unnormalised partial per query instead of out: 132
   // floats {o[128], m, l, pad} at part + query * 132 (m the running maximum in
   // the exp2 domain, l the sum of exp2(s - m), o the sum of exp2(s - m) v)
   int blk0 = 0, blk1 = 0;
   float *part = nullptr;
 };
 
-__device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale, TileLds &sh) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// One online-softmax step of a lane's query over 8 N / 2 raw scores st (16-key
+// rows of S^T, masked to -inf where not visible): updates the running maximum
+// m (of score * qscale) and this lane's part l of the denominator, leaves the
+// three truncated bf16 pieces of p = exp2(score * qscale - m) in pw per 32
+// keys (the top 8, next 8 and last 8 significant bits of p; each remainder is
+// exact, so p is their sum), and returns the factor for the previous O. The
+// scale is applied in the exponent's fma: one rounding less than a scaled
+// score, and one instruction.
+template <int N>
+__device__ __forceinline__ float softmax_step(const f32x4 (&st)[N], float qscale, float &m_run,
+                                              float &l_run, uint32_t (&pw)[N / 2][3][4]) {
+  float mx = st[0][0];
+#pragma unroll
+  for (int e = 1; e < 4 * N; ++e)
+    mx = fmaxf(mx, st[e >> 2][e & 3]);
+  mx = max_halves(max_row_pairs(mx)) * qscale;
+  const float m_new = fmaxf(m_run, mx);
+  const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
+  const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
+  float ps = 0.f;
+#pragma unroll
+  for (int g = 0; g < N / 2; ++g)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 &s = st[2 * g + (q >> 1)];
+      float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * (q & 1)], qscale, -m_use));
+      float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * (q & 1) + 1], qscale, -m_use));
+      ps += p0;
+      ps += p1;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const uint32_t u0 = __builtin_bit_cast(uint32_t, p0);
+        const uint32_t u1 = __builtin_bit_cast(uint32_t, p1);
+        pw[g][k][q] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // hi16(u0) | hi16(u1) << 16
+        p0 -= __builtin_bit_cast(float, u0 & 0xffff0000u);
+        p1 -= __builtin_bit_cast(float, u1 & 0xffff0000u);
+      }
+    }
+  l_run = l_run * corr + ps;
+  m_run = m_new;
+  return corr;
+}
+__device__ __forceinline__ u32x4 piece(const uint32_t (&w)[4]) { return u32x4{w[0], w[1], w[2], w[3]}; }
+
+// A lane's 4 output dims from d of one query row: bf16(o / l).
+__device__ __forceinline__ void store_dims(uint16_t *dst, int d, f32x4 o, float l) {
+  const uint32_t lo = uint32_t(f2bf(o[0] / l)) | (uint32_t(f2bf(o[1] / l)) << 16);
+  const uint32_t hi = uint32_t(f2bf(o[2] / l)) | (uint32_t(f2bf(o[3] / l)) << 16);
+  *reinterpret_cast<uint2 *>(dst + d) = uint2{lo, hi};
+}
+
+typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+// Buffers over a tile's K rows and V: reads past the last key (of V in blocks:
+// past its last block) give zeros; the scores of those keys are masked.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t k_rsrc(const QueryTile &t) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(t.kc), 0, uint32_t(t.kend) * (D * 2),
+                                           0x00020000);
+}
+template <bool kRows>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t v_rsrc(const QueryTile &t) {
+  const int keys = kRows ? t.kend : (((t.kend - 1) >> 5) + 1) * kBlock;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(t.vc), 0, uint32_t(keys) * (D * 2),
+                                           0x00020000);
+}
+
+// V of a 32-key block staged as it lies in memory, 8 KiB either way.
+//
+// Rows ([32 keys][128 dims]): 16-byte chunk c of key R at slot c ^ 2 h(R) of
+// its row, h(R) = R % 4 + 4 (R / 8 % 2). The P.V operand of dim tile dt (lane
+// (i, r): dim 16 dt + i, keys 8 r + [0, 8)) is two transposing reads
+// (ds_read_b64_tr_b16: in each group of 16 lanes, lane 4 a + b gives the
+// address of 4 dims from 4 b of key a and lane j receives dim j of the 4
+// keys), keys 8 r + a and 8 r + 4 + a; the swizzle puts the 8 keys of half a
+// wave in 8 different 32-byte windows.
+__device__ __forceinline__ uint32_t v_row_fetch(int lane, int q) {  // load q's lane offset in bytes
+  const int R = 4 * q + (lane >> 4);
+  return uint32_t(R * (D * 2) + ((lane & 15) ^ (2 * ((R & 3) + 4 * ((R >> 3) & 1)))) * 16);
+}
+__device__ __forceinline__ int v_row_read(int lane, int dt) {  // u32x4 slots x 2 (8-byte units)
+  const int R = 8 * (lane >> 4) + ((lane >> 2) & 3);
+  return R * 32 + ((dt ^ ((R & 3) + 4 * ((R >> 3) & 1))) * 4) + (lane & 3);
+}
+__device__ __forceinline__ u32x4 v_row_operand(const u32x4 *stage, int at) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) s16x4 *lds_s16x4;
+  const u32x2 *p = reinterpret_cast<const u32x2 *>(stage) + at;
+  const u32x2 lo = __builtin_bit_cast(
+      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)const_cast<u32x2 *>(p)));
+  const u32x2 hi = __builtin_bit_cast(  // keys + 4
+      u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)const_cast<u32x2 *>(p + 128)));
+  return u32x4{lo.x, lo.y, hi.x, hi.y};
+}
+// Blocks (dim-major [128 dims][32 keys]): 16-byte chunk c of dim d at slot
+// c ^ (d / 4) % 4 of its 64 bytes; an operand is one 16-byte read.
+__device__ __forceinline__ uint32_t v_block_fetch(int lane, int q) {
+  return uint32_t(q * 1024 + (lane >> 2) * 64 + ((lane & 3) ^ (lane >> 4)) * 16);
+}
+
+// ---------------------------------------------------------------------------
+// Key-split tile of 16 C queries: wave w of W walks the 32-key blocks w,
+// w + W, ... A block's K and V are 8 contiguous KiB each; a wave fetches them
+// into an LDS stage of its own by direct-to-LDS loads of whole KiB and moves
+// them to registers before it refills the stage, so the next block is in
+// flight during the products and no barrier runs before the merge. Loading
+// the MFMA operands straight into registers (16 rows x 64 bytes a load) left a
+// CU at ~45 KB/us, more waves or not; this pulls ~80. Slot p of a stage, K:
+// key p / 16, 16-byte chunk (p % 16) ^ f(key), f = the key's row of its S^T
+// tile; V as above. Operand reads then go to 16 different 16-byte slots per
+// group of lanes (gemm.hip).
+// MI355X, 24/8 heads, us, before (4 waves, registers) -> now: 33 queries after
+// 2000 keys 26.7 -> 13.9, 160 after 600 13.5 -> 8.4, 160 from 0 7.5 -> 5.3, 512
+// from 0 14.1 -> 11.2, 700 after 600 (64-query tiles) 34.4 -> 27.6.
+
+template <int C, int W>
+struct TileLds {
+  u32x4 kv[W][2][512];  // [wave][K | V]; the merge's O lies over it
+  float m[W][C][16], l[W][C][16];
+};
+
+template <int C, bool kRows, int W>
+__device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale,
+                                                TileLds<C, W> &sh) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane >> 4, i = lane & 15;
-  const int nblk = (t.kend + kBlock - 1) / kBlock;
-  const int last = t.kend - 1;
+  const int nblk = t.blk1 ? t.blk1 : (t.kend + kBlock - 1) / kBlock;  // blocks [blk0, nblk)
+  const int first = t.blk0 + wave;
+  const auto rk = k_rsrc(t), rv = v_rsrc<kRows>(t);
+  u32x4 *ks = sh.kv[wave][0], *vs = sh.kv[wave][1];
+  auto fetch = [&](int kb) {
+    const uint32_t base = uint32_t(kb) * (D * 2);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rk, (lds_ptr_t)(ks + 64 * q), 16,
+          base + uint32_t((4 * q + r) * (D * 2) + (i ^ (4 * (q >> 1) + r)) * 16), 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rv, (lds_ptr_t)(vs + 64 * q), 16,
+          base + (kRows ? v_row_fetch(lane, q) : v_block_fetch(lane, q)), 0, 0, 0);
+  };
+  if (first < nblk)
+    fetch(first * kBlock);
 
   // Q^T operands: column tile c, query 16 c + i (clamped), dims 32 s + 8 r
-  u32x4 qb[2][4];
+  u32x4 qb[C][4];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < C; ++c) {
     const int qi = min(16 * c + i, t.nq - 1);
     const u32x4 *src = reinterpret_cast<const u32x4 *>(t.q + size_t(qi) * t.q_stride);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
       qb[c][s] = src[4 * s + r];
   }
-  float m_run[2] = {-__builtin_inff(), -__builtin_inff()}, l_run[2] = {0.f, 0.f};
-  f32x4 o[2][8];
+  float m_run[C], l_run[C];
+  f32x4 o[C][8];
 #pragma unroll
-  for (int c = 0; c < 2; ++c)
+  for (int c = 0; c < C; ++c) {
+    m_run[c] = -__builtin_inff();
+    l_run[c] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
       o[c][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  if (wave < nblk) {  // uniform per wave
-    u32x4 kr[8];
-    load_k(t.kc, wave * kBlock, 0, lane, last, kr);
-    for (int blk = wave; blk < nblk; blk += 4) {
-      const int kb = blk * kBlock;
-      const bool more = blk + 4 < nblk;  // uniform
-      // this block's V lands during S^T and the softmax; the next block's K
-      // is in flight during the whole step (two waves per SIMD hide the rest)
-      u32x4 vr[8], kn[8];
-      load_v(t.vc, kb, 0, lane, last, vr);
-      if (more)
-        load_k(t.kc, kb + 4 * kBlock, 0, lane, last, kn);
+  }
+  auto block = [&](int blk, auto mask_tag) {
+    constexpr bool kMask = decltype(mask_tag)::value;
+    const int kb = blk * kBlock;
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the block has landed
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 kr[8], vr[8];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x4 st[2];
+    for (int j = 0; j < 8; ++j)
+      kr[j] = ks[key_ofs(j >> 2, i) * 16 + ((4 * (j & 3) + r) ^ i)];
 #pragma unroll
-        for (int T = 0; T < 2; ++T) {
-          st[T] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < 8; ++dt)
+      vr[dt] = kRows ? v_row_operand(vs, v_row_read(lane, dt)) : vs[64 * dt + 4 * i + (r ^ (i >> 2))];
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): it is in registers
+    __builtin_amdgcn_sched_barrier(0);
+    if (blk + W < nblk)
+      fetch(kb + W * kBlock);
+    // a score tile's four k-steps depend on each other: the chains of the
+    // tiles are interleaved, and below those of the dim tiles
+    f32x4 st[C][2];
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-            st[T] = mfma(kr[4 * T + s], qb[c][s], st[T]);
-        }
-        // lane (query 16 c + i, r): keys kb + 8 r + 4 T + u
-        const int kmax = t.causal_pos >= 0 ? t.causal_pos + 16 * c + i : t.kv_len - 1;
-        float sc[8];
+    for (int c = 0; c < C; ++c)
+      st[c][0] = st[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int T = 0; T < 2; ++T)
+          st[c][T] = mfma(kr[4 * T + s], qb[c][s], st[c][T]);
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            sc[4 * T + u] = kb + 8 * r + 4 * T + u <= kmax ? st[T][u] * qscale : -__builtin_inff();
-        float mx = sc[0];
+    for (int c = 0; c < C; ++c) {
+      if constexpr (kMask) {  // lane (query 16 c + i, r): keys kb + 8 r + 4 T + u
+        const int kmax = (t.causal_pos >= 0 ? t.causal_pos + 16 * c + i : t.kv_len - 1) - kb - 8 * r;
 #pragma unroll
-        for (int e = 1; e < 8; ++e)
-          mx = fmaxf(mx, sc[e]);
-        mx = max_halves(max_row_pairs(mx));
-        const float m_new = fmaxf(m_run[c], mx);
-        const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
-        const float corr = __builtin_amdgcn_exp2f(m_run[c] - m_use);
-        float ps = 0.f;
-        uint32_t pw[3][4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float p0 = __builtin_amdgcn_exp2f(sc[2 * q] - m_use);
-          float p1 = __builtin_amdgcn_exp2f(sc[2 * q + 1] - m_use);
-          ps += p0;
-          ps += p1;
-          // three truncated bf16 pieces: the top 8, next 8 and last 8
-          // significant bits of p; each remainder is exact, so p is their sum
-#pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            const uint32_t u0 = __builtin_bit_cast(uint32_t, p0);
-            const uint32_t u1 = __builtin_bit_cast(uint32_t, p1);
-            pw[k][q] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // hi16(u0) | hi16(u1) << 16
-            p0 -= __builtin_bit_cast(float, u0 & 0xffff0000u);
-            p1 -= __builtin_bit_cast(float, u1 & 0xffff0000u);
-          }
-        }
-        l_run[c] = l_run[c] * corr + ps;
-        m_run[c] = m_new;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-          o[c][dt] *= corr;
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-            o[c][dt] = mfma(vr[dt], u32x4{pw[k][0], pw[k][1], pw[k][2], pw[k][3]}, o[c][dt]);
-        }
+        for (int e = 0; e < 8; ++e)
+          if (e > kmax)
+            st[c][e >> 2][e & 3] = -__builtin_inff();
       }
-      if (more) {
+      uint32_t pw[1][3][4];
+      const float corr = softmax_step<2>(st[c], qscale, m_run[c], l_run[c], pw);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          kr[j] = kn[j];
-      }
+      for (int dt = 0; dt < 8; ++dt)
+        o[c][dt] *= corr;
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+          o[c][dt] = mfma(vr[dt], piece(pw[0][k]), o[c][dt]);
     }
-  }
+  };
+  // blocks every query of the tile sees in full run without the mask
+  const int kfull = (t.causal_pos >= 0 ? t.causal_pos + 1 : t.kv_len) / kBlock;
+  int blk = first;
+  for (; blk < min(kfull, nblk); blk += W)
+    block(blk, std::false_type{});
+  for (; blk < nblk; blk += W)
+    block(blk, std::true_type{});
 
-  // Merge the four waves' partials: wave w finishes column tile w / 2, dim
-  // tiles 4 (w % 2) .. + 3. A wave that saw no visible key of a query has
-  // m = -inf and weight 0 (key 0 is in wave 0's first block and visible to
-  // every query, so the maximum is finite).
+  // Merge the waves' partials: wave w finishes column tile w / (W / C) and C
+  // of its dim tiles. A wave that saw no visible key of a query has m = -inf
+  // and weight 0 (the range's first key is in wave 0's first block and
+  // visible to every query, so the maximum is finite). Every load of the stages has landed;
+  // past the barrier the merge may use them.
+  __syncthreads();
+  f32x4 *mo = reinterpret_cast<f32x4 *>(&sh.kv[0][0][0]);  // [wave][c][dt][lane]
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < C; ++c) {
     const float l = sum_halves(sum_row_pairs(l_run[c]));
     if (r == 0) {
       sh.m[wave][c][i] = m_run[c];
@@ -163,74 +285,65 @@ __device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale
     }
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
-      sh.o[wave][c][dt][lane] = o[c][dt];
+      mo[((wave * C + c) * 8 + dt) * 64 + lane] = o[c][dt];
   }
   __syncthreads();
-  const int c = wave >> 1, d0 = 4 * (wave & 1);
-  float f[4], M = -__builtin_inff();
+  const int c = wave / (W / C), d0 = (8 * C / W) * (wave % (W / C));
+  float f[W], M = -__builtin_inff();
 #pragma unroll
-  for (int w = 0; w < 4; ++w)
+  for (int w = 0; w < W; ++w)
     M = fmaxf(M, sh.m[w][c][i]);
   float L = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < W; ++w) {
     const float m = sh.m[w][c][i];
     f[w] = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - M);
     L += f[w] * sh.l[w][c][i];
   }
   const int qi = 16 * c + i;
   if (qi < t.nq) {
+    float *pq = t.part ? t.part + size_t(qi) * 132 : nullptr;
+    if (pq && d0 == 0 && r == 0) {
+      pq[128] = M;
+      pq[129] = L;
+    }
     uint16_t *dst = t.out + size_t(qi) * t.out_stride;
 #pragma unroll
-    for (int dt = d0; dt < d0 + 4; ++dt) {
-      f32x4 acc = sh.o[0][c][dt][lane] * f[0];
+    for (int dt = d0; dt < d0 + 8 * C / W; ++dt) {
+      f32x4 acc = mo[(c * 8 + dt) * 64 + lane] * f[0];
 #pragma unroll
-      for (int w = 1; w < 4; ++w)
-        acc += sh.o[w][c][dt][lane] * f[w];
-      // lane (query, r) holds dims 16 dt + 4 r + [0, 4): out = bf16(o / l)
-      const uint32_t lo = uint32_t(f2bf(acc[0] / L)) | (uint32_t(f2bf(acc[1] / L)) << 16);
-      const uint32_t hi = uint32_t(f2bf(acc[2] / L)) | (uint32_t(f2bf(acc[3] / L)) << 16);
-      *reinterpret_cast<uint2 *>(dst + 16 * dt + 4 * r) = uint2{lo, hi};
+      for (int w = 1; w < W; ++w)
+        acc += mo[((w * C + c) * 8 + dt) * 64 + lane] * f[w];
+      // lane (query, r) holds dims 16 dt + 4 r + [0, 4)
+      if (pq)
+        *reinterpret_cast<f32x4 *>(pq + 16 * dt + 4 * r) = acc;
+      else
+        store_dims(dst, 16 * dt + 4 * r, acc, L);
     }
   }
 }
 
 // ---------------------------------------------------------------------------
 // 64-query tile with K/V shared through LDS: wave w owns queries 16 w + i and
-// all four waves walk the same 32-key blocks. Each block's K and V are
+// all four waves walk the same keys, 64 per step (two 32-key blocks: one
+// rescale of O and one cross-lane maximum for both). Each block's K and V are
 // fetched once per workgroup (each wave loads a quarter: K pieces and V dim
-// tiles 2 w, 2 w + 1 in the MFMA operand layout of load_k / load_v) into an
-// LDS ring ahead of the block being computed; every wave then reads its
-// operands from LDS. Same arithmetic per query as
-// attn_query_tile (fp32 scores, exp2 online softmax, P as three truncated
-// bf16 pieces, fp32 sums, bf16(o / l)), with no merge across waves.
-// Workgroups of the 64-query tile below which the 32-query key-split tile
-// is faster on MI355X's 256 CUs (measured, causal self-attention at 24/8
-// heads: 288 workgroups of 64 queries (768 tokens) lose to 576 of 32, 23.3
-// against 22.1 us; 384 (1024 tokens) win, 30.5 against 33.5 us, and the gap
-// grows with the length: 66.6 against 85 us at 1984 tokens).
-constexpr int kTile64MinGroups = 384;
-// Key splits of a non-causal launch aim at this many workgroups.
-constexpr int kSplitTargetGroups = 768;
-
-// LDS ring of two stages (32 KiB: one block ahead), filled by direct-to-LDS
-// loads, so the next block needs no registers: 96 VGPRs, five waves per SIMD
-// and five workgroups per CU (160 KiB of LDS). Three stages with register
-// staging (48 KiB, 131 VGPRs, three waves) measured 2-4% slower than two.
-constexpr int kTile64Stages = 2;
-constexpr int kTile64Waves = 5;  // waves per SIMD (LDS, registers)
-
-struct Tile64Lds {
-  u32x4 k[kTile64Stages][8][64];  // [stage][piece][lane]
-  u32x4 v[kTile64Stages][8][64];
+// tiles 2 w, 2 w + 1 in the MFMA operand layout of load_k / load_v, which the
+// operand reads then find at constant offsets; whole-KiB loads with swizzled
+// reads measured 0-8% slower here) into an LDS ring of two steps, one step
+// ahead; every wave reads its operands from LDS. No merge across waves.
+struct Tile64Lds {  // 64 KiB: two workgroups per CU, two waves per SIMD
+  u32x4 k[2][2][8][64];  // [stage][32-key block][piece][lane]
+  u32x4 v[2][2][8][64];
 };
 
+template <bool kRows>
 __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qscale,
                                                   Tile64Lds &sh) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane >> 4, i = lane & 15;
-  const int b_lo = t.blk0;
-  const int nblk = t.blk1 ? t.blk1 : (t.kend + kBlock - 1) / kBlock;  // blocks [b_lo, nblk)
+  const int nblk = (t.kend + kBlock - 1) / kBlock, nkeys = nblk * kBlock;
   const int last = t.kend - 1;
   u32x4 qb[4];
   {
@@ -241,29 +354,31 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
       qb[s] = src[4 * s + r];
   }
   const int kmax = t.causal_pos >= 0 ? t.causal_pos + 16 * wave + i : t.kv_len - 1;
-  // this wave's quarter of the block at kb into `stage`: K pieces 2 w, 2 w + 1
-  // (T = w / 2, s = 2 (w % 2) + {0, 1}) and V dim tiles 2 w, 2 w + 1, each a
-  // direct-to-LDS buffer load that puts lane l's 16 bytes in slot l of the
-  // piece row (the MFMA operand layout; no registers in between). Keys and
-  // blocks are clamped to the last visible one, inside both ranges.
-  const auto rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(t.kc), 0,
-                                                    uint32_t(t.kend) * (D * 2), 0x00020000);
-  const auto rv = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<u32x4 *>(t.vc), 0, uint32_t((last >> 5) + 1) * (kBlock * D * 2), 0x00020000);
-  auto fetch = [&](int kb, int stage) {
-    const int key = min(kb + key_ofs(wave >> 1, i), last);
-    const uint32_t ko = uint32_t(key * (D / 8) + 8 * (wave & 1) + r) * 16;
-    const uint32_t vo = uint32_t(min(kb >> 5, last >> 5)) * (kBlock * D * 2) +
-                        uint32_t((32 * wave + i) * (kBlock / 8) + r) * 16;
-    typedef __attribute__((address_space(3))) void *lds_ptr_t;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)&sh.k[stage][2 * wave][0], 16, ko, 0,
-                                             0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)&sh.k[stage][2 * wave + 1][0], 16,
-                                             ko + 64, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)&sh.v[stage][2 * wave][0], 16, vo, 0,
-                                             0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)&sh.v[stage][2 * wave + 1][0], 16,
-                                             vo + 16 * kBlock * 2, 0, 0, 0);
+  const auto rk = k_rsrc(t), rv = v_rsrc<kRows>(t);
+  // this wave's quarter of the two blocks at kb0 into `stage`: K pieces 2 w,
+  // 2 w + 1 (T = w / 2, s = 2 (w % 2) + {0, 1}) and V dim tiles 2 w, 2 w + 1.
+  // Keys are clamped to the last visible one.
+  auto fetch = [&](int kb0, int stage) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int kb = kb0 + kBlock * g;
+      const int key = min(kb + key_ofs(wave >> 1, i), last);
+      const uint32_t ko = uint32_t(key * (D / 8) + 8 * (wave & 1) + r) * 16;
+      // the missing half of an odd last step: V past the range, zeros (its
+      // weights are zero, and 0 * inf of another block would be NaN)
+      const uint32_t vb = uint32_t(min(kb, nkeys)) * (D * 2);
+      const uint32_t vo0 = vb + (kRows ? v_row_fetch(lane, 2 * wave)
+                                       : uint32_t((32 * wave + i) * (kBlock / 8) + r) * 16);
+      const uint32_t vo1 = kRows ? vb + v_row_fetch(lane, 2 * wave + 1) : vo0 + 1024;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)&sh.k[stage][g][2 * wave][0], 16, ko,
+                                               0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)&sh.k[stage][g][2 * wave + 1][0], 16,
+                                               ko + 64, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)&sh.v[stage][g][2 * wave][0], 16, vo0,
+                                               0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)&sh.v[stage][g][2 * wave + 1][0], 16,
+                                               vo1, 0, 0, 0);
+    }
   };
 
   float m_run = -__builtin_inff(), l_run = 0.f;
@@ -271,114 +386,138 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt)
     o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int S = kTile64Stages;
-  fetch(b_lo * kBlock, b_lo % S);
+  const int steps = (nblk + 1) / 2;
+  fetch(0, 0);
   __builtin_amdgcn_s_waitcnt(0);  // (a barrier waits for no load)
   __syncthreads();
-  // one block; kMask: the causal / key-length mask, needed only from the
-  // first block with a key past the smallest kmax of the tile's queries (the
-  // blocks before it are visible to every query: same scores, no compares)
-  auto block = [&](int b, auto mask_tag) {
+  // one step of 64 keys; kMask: the causal / key-length mask, needed only from
+  // the first step with a key past the smallest kmax of the tile's queries
+  auto step = [&](int x, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
-    const int stage = b % S, kb = b * kBlock;
-    // block b + 1 into the stage every wave finished reading before the
-    // previous barrier; in flight during this block's products
-    if (b + 1 < nblk)  // uniform
-      fetch(kb + kBlock, (b + 1) % S);
-    u32x4 kr[8];
+    const int stage = x & 1, kb = 2 * x * kBlock;
+    // step x + 1 into the stage every wave finished reading before the
+    // previous barrier; in flight during this step's products
+    if (x + 1 < steps)  // uniform
+      fetch(kb + 2 * kBlock, stage ^ 1);
+    // four independent chains of four dependent MFMAs, interleaved
+    f32x4 st[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      kr[j] = sh.k[stage][j][lane];
-    f32x4 st[2];
+    for (int j = 0; j < 4; ++j)
+      st[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int T = 0; T < 2; ++T) {
-      st[T] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-        st[T] = mfma(kr[4 * T + s], qb[s], st[T]);
+      for (int j = 0; j < 4; ++j)
+        st[j] = mfma(sh.k[stage][j >> 1][4 * (j & 1) + s][lane], qb[s], st[j]);
+    if constexpr (kMask) {  // lane (query 16 w + i, r): keys kb + 32 g + 8 r + 4 T + u
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (kb + 32 * (e >> 3) + 8 * r + (e & 7) > kmax)
+          st[e >> 2][e & 3] = -__builtin_inff();
     }
-    // lane (query 16 w + i, r): keys kb + 8 r + 4 T + u
-    float sc[8];
-#pragma unroll
-    for (int T = 0; T < 2; ++T)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        sc[4 * T + u] = !kMask || kb + 8 * r + 4 * T + u <= kmax ? st[T][u] * qscale
-                                                                : -__builtin_inff();
-    float mx = sc[0];
-#pragma unroll
-    for (int e = 1; e < 8; ++e)
-      mx = fmaxf(mx, sc[e]);
-    mx = max_halves(max_row_pairs(mx));
-    const float m_new = fmaxf(m_run, mx);
-    const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
-    const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
-    float ps = 0.f;
-    uint32_t pw[3][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float p0 = __builtin_amdgcn_exp2f(sc[2 * q] - m_use);
-      float p1 = __builtin_amdgcn_exp2f(sc[2 * q + 1] - m_use);
-      ps += p0;
-      ps += p1;
-      // three truncated bf16 pieces: the top 8, next 8 and last 8
-      // significant bits of p; each remainder is exact, so p is their sum
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const uint32_t u0 = __builtin_bit_cast(uint32_t, p0);
-        const uint32_t u1 = __builtin_bit_cast(uint32_t, p1);
-        pw[k][q] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // hi16(u0) | hi16(u1) << 16
-        p0 -= __builtin_bit_cast(float, u0 & 0xffff0000u);
-        p1 -= __builtin_bit_cast(float, u1 & 0xffff0000u);
-      }
-    }
-    l_run = l_run * corr + ps;
-    m_run = m_new;
-    u32x4 vr[8];
+    uint32_t pw[2][3][4];
+    const float corr = softmax_step<4>(st, qscale, m_run, l_run, pw);
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
-      vr[dt] = sh.v[stage][dt][lane];
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
       o[dt] *= corr;
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        o[dt] = mfma(vr[dt], u32x4{pw[k][0], pw[k][1], pw[k][2], pw[k][3]}, o[dt]);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of block b + 1
-    __syncthreads();
-  };
-  const int kfull = (t.causal_pos >= 0 ? t.causal_pos + 1 : t.kv_len) / kBlock;
-  int b = b_lo;
-  for (; b < min(kfull, nblk); ++b)
-    block(b, std::false_type{});
-  for (; b < nblk; ++b)
-    block(b, std::true_type{});
-  // lane (query 16 w + i, r) holds dims 16 dt + 4 r + [0, 4): out = bf16(o / l)
-  const float L = sum_halves(sum_row_pairs(l_run));
-  const int qi = 16 * wave + i;
-  if (t.part) {
-    if (qi < t.nq) {
-      float *pq = t.part + size_t(qi) * 132;
+    for (int g = 0; g < 2; ++g) {
+      u32x4 vr[8];
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
-        *reinterpret_cast<f32x4 *>(pq + 16 * dt + 4 * r) = o[dt];
-      if (r == 0) {
-        pq[128] = m_run;
-        pq[129] = L;
-      }
-    }
-    return;
-  }
-  if (qi < t.nq) {
-    uint16_t *dst = t.out + size_t(qi) * t.out_stride;
+        vr[dt] = kRows ? v_row_operand(sh.v[stage][g][0], v_row_read(lane, dt))
+                       : sh.v[stage][g][dt][lane];
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const uint32_t lo = uint32_t(f2bf(o[dt][0] / L)) | (uint32_t(f2bf(o[dt][1] / L)) << 16);
-      const uint32_t hi = uint32_t(f2bf(o[dt][2] / L)) | (uint32_t(f2bf(o[dt][3] / L)) << 16);
-      *reinterpret_cast<uint2 *>(dst + 16 * dt + 4 * r) = uint2{lo, hi};
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+          o[dt] = mfma(vr[dt], piece(pw[g][k]), o[dt]);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of step x + 1
+    __syncthreads();
+  };
+  const int kfull = t.causal_pos >= 0 ? t.causal_pos + 1 : t.kv_len;
+  int x = 0;
+  for (; x < min(kfull / (2 * kBlock), steps); ++x)
+    step(x, std::false_type{});
+  for (; x < steps; ++x)
+    step(x, std::true_type{});
+  // lane (query 16 w + i, r) holds dims 16 dt + 4 r + [0, 4)
+  const float L = sum_halves(sum_row_pairs(l_run));
+  const int qi = 16 * wave + i;
+  if (qi >= t.nq)
+    return;
+  uint16_t *dst = t.out + size_t(qi) * t.out_stride;
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt)
+    store_dims(dst, 16 * dt + 4 * r, o[dt], L);
+}
+
+// How a launch of `heads` heads (batch included) x q_len queries over kv_len
+// keys is cut: queries and waves per workgroup (64: attn_query_tile64, else
+// the key-split tile) and, where the keys may be dealt (non-causal, key-split),
+// groups > 0: the steps of all tiles, `waves` key blocks each, go to that many
+// workgroups in equal contiguous runs, merged by another kernel. (64-query
+// tiles dealt gave no more than the 32-query ones: 512 x 3512, 24 heads, 57 and
+// 57 us.)
+//
+// By a time model in us, fitted on MI355X's 256 CUs at 24/8 and 16/8 heads to
+// 90 non-causal shapes (33-1024 queries x 400-8000 keys) and 150 causal ones
+// (9-3000 queries after 0-2000 keys), every form timed: the pick is within
+// 0.8% of the fastest form on average (10% at worst) and takes 0.72 of the
+// time of the forms before (32 queries by 4 waves from registers; 64 queries,
+// ranges of keys for up to 768 workgroups). A round of workgroups costs
+// `launch`; a step costs `alone` where a workgroup has a CU to itself and
+// `shared` (`causal`: tiles of unequal length) where two do, eight waves
+// always; a further tile of a dealt run 0.8; the merge 5.0 and 0.35 per MB of
+// partials.
+struct TilePlan {
+  int queries = 64, waves = 4, groups = 0;
+};
+constexpr int kMaxPieces = 16;  // workgroups that may hold parts of a dealt tile
+inline TilePlan attn_tile_plan(long long heads, int q_len, int kv_len, bool causal, bool deal) {
+  struct Form {
+    int queries, waves;
+    double launch, alone, shared, causal;
+  };
+  static const Form forms[] = {{16, 4, 3.3, 0.82, 1.30, 1.24}, {16, 8, 4.3, 1.18, 1.18, 1.31},
+                               {32, 4, 4.4, 1.13, 1.99, 1.52}, {32, 8, 5.3, 1.98, 1.98, 1.96},
+                               {64, 4, 4.4, 1.20, 2.02, 1.24}};
+  const int nb = (kv_len + kBlock - 1) / kBlock;
+  TilePlan best;
+  double best_t = __builtin_inf();
+  auto take = [&](const Form &f, int groups, double t) {
+    if (t < best_t) {
+      best = TilePlan{f.queries, f.waves, groups};
+      best_t = t;
+    }
+  };
+  for (const Form &f : forms) {
+    const int blocks = f.queries == 64 ? 2 : f.waves, slots = f.waves == 8 ? 256 : 512;
+    const long long tiles = heads * ((q_len + f.queries - 1) / f.queries);
+    const long long steps = (nb + blocks - 1) / blocks, total = tiles * steps;
+    const double busy = causal ? f.causal : f.shared, alone = f.waves == 8 ? busy : f.alone;
+    // past three rounds the key-split tiles lose to the 64-query one (3000
+    // queries after 0 keys, 16 heads: 85 against 77 us)
+    if (f.queries == 64 || tiles <= 1536) {
+      const double mean =
+          causal ? (nb - std::max(0, q_len - f.queries) / 64.0) / blocks : double(steps);
+      const long long rem = tiles % slots;
+      const double rate =
+          double(tiles / slots) * busy + (rem == 0 ? 0.0 : rem <= 256 ? alone : busy);
+      take(f, 0, f.launch * double((tiles + slots - 1) / slots) +
+                     std::max((tiles <= 256 ? alone : busy) * double(steps), rate * mean));
+    }
+    // dealt: at least two steps a workgroup, at most kMaxPieces pieces a tile
+    // (and total * slots in 31 bits, which the kernels count in)
+    if (deal && !causal && f.queries < 64 && total >= 2 * slots && total < (1 << 21) &&
+        (steps - 1) / (total / slots) + 2 <= kMaxPieces) {
+      const double mb = double(slots + std::min<long long>(slots, tiles)) * f.queries * (132 * 4e-6);
+      take(f, slots, f.launch + 0.8 * double(tiles) / slots +
+                         f.shared * double((total + slots - 1) / slots) + 5.0 + 0.35 * mb);
     }
   }
+  return best;
 }
 
 }  // namespace attn

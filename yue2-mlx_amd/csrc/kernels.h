@@ -107,22 +107,19 @@ int attn_decode_splits(int batch, int kv_heads, int kv_stride);
 
 // Acoustic-model attention (nar_attention.hip, nar_attention.cpp:63-270):
 // q [batch][heads][q_len][128], k / v [batch][kv_heads][kv_len][128], out
-// like q; vb: workspace of nar_attention_workspace_elems() bf16 (V in 32-key
-// dim-major blocks). causal needs q_len == kv_len.
+// like q. causal needs q_len == kv_len.
 struct NarAttnParams {
   const uint16_t *q = nullptr, *k = nullptr, *v = nullptr;
-  uint16_t *vb = nullptr;
   uint16_t *out = nullptr;
   int batch = 1, heads = 0, kv_heads = 0, q_len = 0, kv_len = 0, causal = 0;
-  int kv_pad = 0;  // set by launch_nar_attention: kv_len rounded up to 32
-  // optional split-key scratch (nar_attention_part_floats() floats): with it,
-  // launches too small to fill the GPU split the keys over workgroups
+  // optional scratch (nar_attention_part_floats() floats): with it, launches
+  // that gain by it deal the keys of a tile to several workgroups
   float *part = nullptr;
   size_t part_floats = 0;
-  int splits = 1;  // set by launch_nar_attention
+  int groups = 0;  // set by launch_nar_attention
 };
-// Floats of split-key partials that let launch_nar_attention split this
-// launch's keys (0: it never splits this shape).
+// Floats of partials that let launch_nar_attention deal this launch's keys (0:
+// it never does for this shape).
 size_t nar_attention_part_floats(int batch, int heads, int q_len, int kv_len, int causal);
 size_t nar_attention_workspace_elems(int batch, int kv_heads, int kv_len);
 // Keys [0, n) of `heads` cache heads (V in 32-key dim-major blocks, heads

@@ -10,12 +10,12 @@
 // fp32 sums, bf16(o / l). causal (Lq == Lk, the conditioning prefill of
 // nar.cpp:176) hides the keys after each query's own position.
 //
-// Structure: one workgroup per (batch, q head, 32-query tile); its 4 waves
-// split the keys and merge in LDS (attn_tile.h, shared with the causal
-// prefill attention). K is read row-major as given. The V^T operand wants 8 consecutive keys of one dim per lane, so V is first
-// rewritten (nar_v_blocks_kernel) into 32-key blocks stored dim-major, the
-// layout of the KV cache, in a caller-provided workspace; keys past Lk in the
-// last block are zero there (and masked in the scores).
+// Structure: the query tiles of attn_tile.h (shared with the causal prefill
+// attention) as attn_tile_plan chooses; non-causal launches may deal the keys
+// of their tiles to a full chip of workgroups, merged by a second kernel. K and
+// V are read as given, V through transposing LDS reads. (Rewriting V into
+// dim-major blocks first makes the 64-query tile 2-5% faster, but cost 5 us a
+// call: 512 x 3512, 24 heads, 57 against 55 us; 1024 x 8000 198 against 198.)
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -33,49 +33,16 @@ using attn::D;
 using attn::f32x4;
 using attn::kBlock;
 
-// One 32-key block of one (batch, kv head): [32][128] row-major in, [128][32]
-// out, through an LDS tile (rows padded to 136 elements: 272-byte rows keep
-// the 16-byte stores aligned and spread the column reads over the banks).
-__global__ __launch_bounds__(256) void nar_v_blocks_kernel(const uint16_t *v, int lk, int lkp,
-                                                           uint16_t *vb) {
-  __shared__ __align__(16) uint16_t tile[kBlock][D + 8];
-  const size_t head = blockIdx.y;
-  const int t0 = blockIdx.x * kBlock;
-  for (int c = threadIdx.x; c < kBlock * D / 8; c += 256) {
-    const int t = c / (D / 8), d8 = (c % (D / 8)) * 8;
-    u32x4 val{0u, 0u, 0u, 0u};
-    if (t0 + t < lk)
-      val = *reinterpret_cast<const u32x4 *>(v + (head * lk + t0 + t) * D + d8);
-    *reinterpret_cast<u32x4 *>(&tile[t][d8]) = val;
-  }
-  __syncthreads();
-  uint16_t *dst = vb + (head * lkp + t0) * D;
-  for (int c = threadIdx.x; c < kBlock * D / 8; c += 256) {
-    const int d = c / (kBlock / 8), k8 = (c % (kBlock / 8)) * 8;
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      w[j] = uint32_t(tile[k8 + 2 * j][d]) | (uint32_t(tile[k8 + 2 * j + 1][d]) << 16);
-    *reinterpret_cast<u32x4 *>(dst + d * kBlock + k8) = u32x4{w[0], w[1], w[2], w[3]};
-  }
-}
-
-// T64: the 64-query tile with K/V shared through LDS (attn_query_tile64),
-// chosen when it yields enough workgroups to fill the GPU; otherwise the
-// 32-query tile whose four waves split the keys.
-template <bool T64>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T64 ? attn::kTile64Waves : 2, T64 ? attn::kTile64Waves : 2))) void nar_attn_kernel(NarAttnParams p, float qscale) {
-  constexpr int kQ = T64 ? 64 : 32;  // queries per workgroup
-  __shared__ std::conditional_t<T64, attn::Tile64Lds, attn::TileLds> sh;
-  const int bh = blockIdx.x;  // batch * heads + head
+// Tile `tile` of kQ queries of one (batch, head).
+template <int kQ>
+__device__ __forceinline__ attn::QueryTile nar_tile(const NarAttnParams &p, int bh, int tile) {
   const int h = bh % p.heads, b = bh / p.heads;
-  const int tile = p.causal ? gridDim.y - 1 - blockIdx.y : blockIdx.y;  // causal: longest first
   const int q0 = tile * kQ;
   const int kvh = h / (p.heads / p.kv_heads);
   const size_t kvhead = size_t(b) * p.kv_heads + kvh;
   attn::QueryTile t;
   t.kc = reinterpret_cast<const u32x4 *>(p.k) + kvhead * p.kv_len * (D / 8);
-  t.vc = reinterpret_cast<const u32x4 *>(p.vb) + kvhead * p.kv_pad * (D / 8);
+  t.vc = reinterpret_cast<const u32x4 *>(p.v) + kvhead * p.kv_len * (D / 8);
   t.nq = min(kQ, p.q_len - q0);
   t.kv_len = p.kv_len;
   t.kend = p.causal ? q0 + t.nq : p.kv_len;
@@ -84,50 +51,107 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T64 ? attn:
   t.q_stride = D;
   t.out = p.out + (size_t(bh) * p.q_len + q0) * D;
   t.out_stride = D;
-  if constexpr (T64) {
-    if (p.splits > 1) {  // keys split over gridDim.z workgroups (non-causal)
-      const int nb = (p.kv_len + attn::kBlock - 1) / attn::kBlock;
-      const int per = (nb + p.splits - 1) / p.splits;
-      t.blk0 = int(blockIdx.z) * per;
-      t.blk1 = min(nb, t.blk0 + per);
-      t.part = p.part + (size_t(blockIdx.z) * p.batch * p.heads * p.q_len +
-                         size_t(bh) * p.q_len + q0) * 132;
-    }
-    attn::attn_query_tile64(t, qscale, sh);
-  } else
-    attn::attn_query_tile(t, qscale, sh);
+  return t;
+}
+
+// The tiles of a workgroup. A dealt launch (p.groups > 0, non-causal): the
+// steps of all tiles (W key blocks each, tile by tile, a head's tiles
+// together) are cut into p.groups equal runs, one per workgroup, so the chip is
+// as full at the end as at the start whatever the number of tiles: 700 x 3512,
+// 24 heads (528 tiles of 32 on 512 slots) 87 -> 75 us against 64-query tiles
+// over equal ranges of keys. A run's part of a tile that it does not hold whole
+// leaves a partial in the workgroup's slot 2 g (the part begins within the
+// tile) or 2 g + 1 (it begins the tile). Workgroup b takes run (b % 8) * groups
+// / 8 + b / 8: an XCD's workgroups take neighbouring runs, whose heads share K
+// and V in its L2.
+template <int kQ, int W, class F>
+__device__ __forceinline__ void nar_run(const NarAttnParams &p, F &&tile_fn) {
+  if (p.groups == 0) {
+    const int tile = p.causal ? gridDim.y - 1 - blockIdx.y : blockIdx.y;  // longest first
+    tile_fn(nar_tile<kQ>(p, blockIdx.x, tile));
+    return;
+  }
+  const int per_head = (p.q_len + kQ - 1) / kQ, nb = (p.kv_len + kBlock - 1) / kBlock;
+  const int steps = (nb + W - 1) / W;  // per tile
+  const int total = p.batch * p.heads * per_head * steps;  // total * groups < 2^31
+  const int g = int(blockIdx.x % 8) * (p.groups / 8) + int(blockIdx.x / 8);
+  const int end = total * (g + 1) / p.groups;
+  for (int s = total * g / p.groups; s < end;) {
+    const int tile = s / steps, x0 = s - tile * steps, x1 = min(steps, x0 + end - s);
+    attn::QueryTile t = nar_tile<kQ>(p, tile / per_head, tile % per_head);
+    t.blk0 = x0 * W;
+    t.blk1 = min(nb, x1 * W);
+    if (x1 - x0 < steps)
+      t.part = p.part + size_t(2 * g + (x0 == 0)) * (kQ * 132);
+    tile_fn(t);
+    s += x1 - x0;
+  }
+}
+// 16 C queries per workgroup, keys split over its waves.
+template <int C, int W>
+__global__ __launch_bounds__(W * 64)
+__attribute__((amdgpu_waves_per_eu(2, 2))) void nar_attn_kernel(NarAttnParams p, float qscale) {
+  __shared__ attn::TileLds<C, W> sh;
+  nar_run<16 * C, W>(p, [&](const attn::QueryTile &t) {
+    attn::attn_query_tile<C, true, W>(t, qscale, sh);
+    __syncthreads();  // the merge has read the stages
+  });
+}
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2))) void nar_attn64_kernel(NarAttnParams p, float qscale) {
+  __shared__ attn::Tile64Lds sh;
+  const int tile = p.causal ? gridDim.y - 1 - blockIdx.y : blockIdx.y;  // longest first
+  attn::attn_query_tile64<true>(nar_tile<64>(p, blockIdx.x, tile), qscale, sh);
 }
 
 // out[row][d] = bf16(sum_s w_s o_s[d] / sum_s w_s l_s), w_s = exp2(m_s - max m)
-// over the split partials of each query row; one thread per (row, 4 dims).
-__global__ __launch_bounds__(256) void nar_merge_kernel(const float *part, int splits, long long rows,
-                                                        uint16_t *out) {
+// over the up to kPieces partials of each query row of a tile that more than
+// one workgroup holds; one thread per (row, 4 dims). All of a thread's loads
+// are issued before the first use (a piece it lacks is read as its last one,
+// with weight 0).
+template <int kPieces>
+__global__ __launch_bounds__(256) void nar_merge_kernel(NarAttnParams p, int kq, int steps,
+                                                        int per_head, int total) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= rows * 32)
+  const int row = int(idx / 32);
+  if (row >= p.batch * p.heads * p.q_len)
     return;
-  const long long row = idx / 32;
   const int d4 = int(idx % 32) * 4;
-  float M = -__builtin_inff();
-  for (int s = 0; s < splits; ++s)
-    M = fmaxf(M, part[(s * rows + row) * 132 + 128]);
-  float L = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < splits; ++s) {
-    const float *ps = part + (s * rows + row) * 132;
-    const float m = ps[128];
-    const float w = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - M);
-    L += w * ps[129];
-    const f32x4 v = *reinterpret_cast<const f32x4 *>(ps + d4);
+  const int bh = row / p.q_len, q = row - bh * p.q_len;
+  const int tile = bh * per_head + q / kq;
+  // workgroup w holds step s: w * total / groups <= s
+  const int w0 = ((tile * steps + 1) * p.groups + total - 1) / total - 1;
+  const int w1 = ((tile + 1) * steps * p.groups + total - 1) / total - 1;
+  const int n = w1 - w0;  // pieces after the first
+  if (n == 0)
+    return;
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  f32x2 ml[kPieces];
+  f32x4 v[kPieces];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] += w * v[j];
+  for (int s = 0; s < kPieces; ++s) {
+    const float *ps =
+        p.part + (size_t(2 * (w0 + min(s, n)) + (s == 0)) * kq + q % kq) * 132;
+    ml[s] = *reinterpret_cast<const f32x2 *>(ps + 128);
+    v[s] = *reinterpret_cast<const f32x4 *>(ps + d4);
   }
-  const uint32_t lo = uint32_t(f2bf(o[0] / L)) | (uint32_t(f2bf(o[1] / L)) << 16);
-  const uint32_t hi = uint32_t(f2bf(o[2] / L)) | (uint32_t(f2bf(o[3] / L)) << 16);
-  *reinterpret_cast<uint2 *>(out + row * 128 + d4) = uint2{lo, hi};
+  float M = ml[0].x;
+#pragma unroll
+  for (int s = 1; s < kPieces; ++s)
+    M = fmaxf(M, ml[s].x);
+  float L = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kPieces; ++s) {
+    const float w = s > n || ml[s].x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - M);
+    L += w * ml[s].y;
+    o += w * v[s];
+  }
+  attn::store_dims(p.out + size_t(row) * D, d4, o, L);
 }
 
-// Inverse of nar_v_blocks_kernel for a cache head: keys [0, n) of each head
-// (blocked, kv_stride slots apart) -> row-major [heads][n][128]; one thread
+// Keys [0, n) of each cache head (V in 32-key dim-major blocks, kv_stride slots
+// apart) -> row-major [heads][n][128]; one thread
 // per 8 dims of one key.
 __global__ __launch_bounds__(256) void v_rows_kernel(const uint16_t *vb, int kv_stride, int heads,
                                                      int n, uint16_t *out) {
@@ -159,26 +183,16 @@ hipError_t launch_v_rows(const uint16_t *vb, int kv_stride, int heads, int n, ui
 }
 
 namespace {
-// Key splits for a non-causal launch whose 64-query workgroups do not fill
-// the GPU: enough to reach kSplitTargetGroups, each split at least 8 blocks.
-// The kernel gives split z the blocks [z * per, min(nb, (z + 1) * per)),
-// per = ceil(nb / splits); the count is recomputed from per so that no
-// split is left without blocks (nb 81 over 10 splits: per 9, 9 splits).
-int nar_splits(int batch, int heads, int q_len, int kv_len, int causal) {
-  const long long g64 = (long long)batch * heads * ((q_len + 63) / 64);
-  const int nb = (kv_len + attn::kBlock - 1) / attn::kBlock;
-  if (causal || g64 >= attn::kSplitTargetGroups)
-    return 1;
-  const int want = int((attn::kSplitTargetGroups + g64 - 1) / g64);
-  const int s = std::max(1, std::min(want, nb / 8));
-  const int per = (nb + s - 1) / s;
-  return (nb + per - 1) / per;
+attn::TilePlan nar_plan(int batch, int heads, int q_len, int kv_len, int causal, bool deal) {
+  return attn::attn_tile_plan((long long)batch * heads, q_len, kv_len, causal != 0, deal);
+}
+size_t part_floats(const attn::TilePlan &plan) {  // two slots per workgroup
+  return size_t(plan.groups) * 2 * plan.queries * 132;
 }
 }  // namespace
 
 size_t nar_attention_part_floats(int batch, int heads, int q_len, int kv_len, int causal) {
-  const int s = nar_splits(batch, heads, q_len, kv_len, causal);
-  return s > 1 ? size_t(s) * batch * heads * q_len * 132 : 0;
+  return part_floats(nar_plan(batch, heads, q_len, kv_len, causal, true));
 }
 
 size_t nar_attention_workspace_elems(int batch, int kv_heads, int kv_len) {
@@ -187,38 +201,39 @@ size_t nar_attention_workspace_elems(int batch, int kv_heads, int kv_len) {
 
 hipError_t launch_nar_attention(NarAttnParams p, hipStream_t s) {
   if (p.batch < 1 || p.heads < 1 || p.kv_heads < 1 || p.heads % p.kv_heads || p.q_len < 1 ||
-      p.kv_len < 1 || (p.causal && p.q_len != p.kv_len) || !p.q || !p.k || !p.v || !p.vb ||
-      !p.out)
+      p.kv_len < 1 || (p.causal && p.q_len != p.kv_len) || !p.q || !p.k || !p.v || !p.out)
     return hipErrorInvalidValue;
-  p.kv_pad = (p.kv_len + kBlock - 1) / kBlock * kBlock;
-  hipLaunchKernelGGL(nar_v_blocks_kernel, dim3(p.kv_pad / kBlock, p.batch * p.kv_heads), dim3(256),
-                     0, s, p.v, p.kv_len, p.kv_pad, p.vb);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess)
-    return e;
   // scale * log2(e) as in the reference kernel (nar_attention.cpp:95)
   const float qscale = 0.08838834764831845f * 1.4426950408889634f;
-  const int splits = nar_splits(p.batch, p.heads, p.q_len, p.kv_len, p.causal);
-  if (splits > 1 && p.part &&
-      p.part_floats >= nar_attention_part_floats(p.batch, p.heads, p.q_len, p.kv_len, p.causal)) {
-    p.splits = splits;
-    hipLaunchKernelGGL(nar_attn_kernel<true>, dim3(p.batch * p.heads, (p.q_len + 63) / 64, splits),
-                       dim3(256), 0, s, p, qscale);
-    e = hipGetLastError();
-    if (e != hipSuccess)
-      return e;
-    const long long rows = (long long)p.batch * p.heads * p.q_len;
-    hipLaunchKernelGGL(nar_merge_kernel, dim3(unsigned((rows * 32 + 255) / 256)), dim3(256), 0, s,
-                       p.part, splits, rows, p.out);
-    return hipGetLastError();
-  }
-  p.splits = 1;
-  if (p.batch * p.heads * ((p.q_len + 63) / 64) >= attn::kTile64MinGroups)
-    hipLaunchKernelGGL(nar_attn_kernel<true>, dim3(p.batch * p.heads, (p.q_len + 63) / 64),
-                       dim3(256), 0, s, p, qscale);
+  attn::TilePlan plan = nar_plan(p.batch, p.heads, p.q_len, p.kv_len, p.causal, true);
+  if (plan.groups && (!p.part || p.part_floats < part_floats(plan)))
+    plan = nar_plan(p.batch, p.heads, p.q_len, p.kv_len, p.causal, false);
+  p.groups = plan.groups;
+  const int heads = p.batch * p.heads, per_head = (p.q_len + plan.queries - 1) / plan.queries;
+  const dim3 grid = plan.groups ? dim3(plan.groups) : dim3(heads, per_head);
+  const dim3 threads(64 * plan.waves);
+  if (plan.queries == 16 && plan.waves == 4)
+    hipLaunchKernelGGL((nar_attn_kernel<1, 4>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 16)
+    hipLaunchKernelGGL((nar_attn_kernel<1, 8>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 32 && plan.waves == 4)
+    hipLaunchKernelGGL((nar_attn_kernel<2, 4>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 32)
+    hipLaunchKernelGGL((nar_attn_kernel<2, 8>), grid, threads, 0, s, p, qscale);
   else
-    hipLaunchKernelGGL(nar_attn_kernel<false>, dim3(p.batch * p.heads, (p.q_len + 31) / 32),
-                       dim3(256), 0, s, p, qscale);
+    hipLaunchKernelGGL(nar_attn64_kernel, grid, threads, 0, s, p, qscale);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !plan.groups)
+    return e;
+  const int nb = (p.kv_len + kBlock - 1) / kBlock;
+  const int steps = (nb + plan.waves - 1) / plan.waves, total = heads * per_head * steps;
+  const int pieces = (steps - 1) / (total / plan.groups) + 2;  // at most
+  const dim3 mgrid(unsigned(((long long)heads * p.q_len * 32 + 255) / 256));
+  auto merge = pieces <= 2   ? nar_merge_kernel<2>
+               : pieces <= 4 ? nar_merge_kernel<4>
+               : pieces <= 8 ? nar_merge_kernel<8>
+                             : nar_merge_kernel<attn::kMaxPieces>;
+  hipLaunchKernelGGL(merge, mgrid, dim3(256), 0, s, p, plan.queries, steps, per_head, total);
   return hipGetLastError();
 }
 

@@ -204,19 +204,14 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(QkPrepParams p) {
 
 // ---------------------------------------------------------------------------
 // Causal attention on MFMA (ar.cpp:284-291: fp32 scores, softmax and P.V,
-// bf16 output): one workgroup per (q head, 32-query tile), the tile's keys
-// [0, pos0 + last query] split over the 4 waves and merged in LDS
-// (attn_tile.h). Query t sits at position pos0 + t. Tiles are dispatched
-// longest causal range first, and all heads of a tile run together so the
-// K/V blocks are shared in L2.
+// bf16 output): one workgroup per (q head, tile of 16, 32 or 64 queries), the
+// forms of attn_tile.h as attn_tile_plan chooses. Query t sits at position
+// pos0 + t and sees keys [0, pos0 + t]. Tiles are dispatched longest causal
+// range first, and all heads of a tile run together so the K/V blocks are
+// shared in L2.
 // ---------------------------------------------------------------------------
-// T64: the 64-query tile with K/V shared through LDS (attn_query_tile64),
-// chosen when it yields enough workgroups to fill the GPU; otherwise the
-// 32-query tile whose four waves split the keys.
-template <bool T64>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T64 ? attn::kTile64Waves : 2, T64 ? attn::kTile64Waves : 2))) void attn_prefill_kernel(AttnPrefillParams p, float qscale) {
-  constexpr int kQ = T64 ? 64 : 32;  // queries per workgroup
-  __shared__ std::conditional_t<T64, attn::Tile64Lds, attn::TileLds> sh;
+template <int kQ>
+__device__ __forceinline__ attn::QueryTile prefill_tile(const AttnPrefillParams &p) {
   using attn::D;
   const int h = blockIdx.x;
   const int tile = gridDim.y - 1 - blockIdx.y;  // longest causal range first
@@ -232,10 +227,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T64 ? attn:
   t.q_stride = size_t(p.heads) * D;
   t.out = p.out + (size_t(q0) * p.heads + h) * D;
   t.out_stride = size_t(p.heads) * D;
-  if constexpr (T64)
-    attn::attn_query_tile64(t, qscale, sh);
-  else
-    attn::attn_query_tile(t, qscale, sh);
+  return t;
+}
+// 16 C queries per workgroup, keys split over its waves.
+template <int C, int W>
+__global__ __launch_bounds__(W * 64)
+__attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(AttnPrefillParams p,
+                                                                    float qscale) {
+  __shared__ attn::TileLds<C, W> sh;
+  attn::attn_query_tile<C, false, W>(prefill_tile<16 * C>(p), qscale, sh);
+}
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill64_kernel(AttnPrefillParams p,
+                                                                      float qscale) {
+  __shared__ attn::Tile64Lds sh;
+  attn::attn_query_tile64<false>(prefill_tile<64>(p), qscale, sh);
 }
 
 }  // namespace
@@ -272,12 +278,19 @@ hipError_t launch_attn_prefill(const AttnPrefillParams &p, hipStream_t s) {
       p.capacity % attn::kBlock)
     return hipErrorInvalidValue;
   const float qscale = float(std::pow(128.0, -0.5)) * 1.4426950408889634f;
-  if (p.heads * ((p.tokens + 63) / 64) >= attn::kTile64MinGroups)
-    hipLaunchKernelGGL(attn_prefill_kernel<true>, dim3(p.heads, (p.tokens + 63) / 64), dim3(256),
-                       0, s, p, qscale);
+  const attn::TilePlan plan =
+      attn::attn_tile_plan(p.heads, p.tokens, p.pos0 + p.tokens, true, false);
+  const dim3 grid(p.heads, (p.tokens + plan.queries - 1) / plan.queries), threads(64 * plan.waves);
+  if (plan.queries == 16 && plan.waves == 4)
+    hipLaunchKernelGGL((attn_prefill_kernel<1, 4>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 16)
+    hipLaunchKernelGGL((attn_prefill_kernel<1, 8>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 32 && plan.waves == 4)
+    hipLaunchKernelGGL((attn_prefill_kernel<2, 4>), grid, threads, 0, s, p, qscale);
+  else if (plan.queries == 32)
+    hipLaunchKernelGGL((attn_prefill_kernel<2, 8>), grid, threads, 0, s, p, qscale);
   else
-    hipLaunchKernelGGL(attn_prefill_kernel<false>, dim3(p.heads, (p.tokens + 31) / 32), dim3(256),
-                       0, s, p, qscale);
+    hipLaunchKernelGGL(attn_prefill64_kernel, grid, dim3(256), 0, s, p, qscale);
   return hipGetLastError();
 }
 
