@@ -236,9 +236,10 @@ yuear_status yuear_session_time_kernel(yuear_session *session,
 
 /* ---- op-level entry points (model_ops, ar.hpp:8-19), device pointers,
  * `stream` is a hipStream_t (NULL = default stream). Scratch memory (the
- * batched GEMV's staging rows, the decode attention's split partials and
- * arrival counters, the split-K GEMM's partials) is per (device, stream):
- * calls on different streams never share it. The first call on a stream (or
+ * staging rows of a batched normed GEMV whose y overlaps x or whose k exceeds
+ * 3072, the decode attention's split partials and arrival counters, the split-K
+ * GEMM's partials) is per (device, stream): calls on different streams never
+ * share it. The first call on a stream (or
  * one needing a larger buffer) allocates, so make it outside graph capture;
  * yuear_op_gemm and yuear_op_gemm_tile use no scratch. The first SwiGLU
  * GEMM (residual 2) on a device fills a 128 KiB silu table (one launch and a

@@ -101,6 +101,31 @@ def test_gemv_matches_oracle(torch, yuear_lib, oracle, n, k, batch, norm, epilog
     assert_close_bf16(got, ref, scale=scale, exact_frac=0.9)
 
 
+@pytest.mark.parametrize("n,k,batch,norm,epilogue", [
+    # batched rows, the edges of the tiles (8 rows) a workgroup holds: one, two,
+    # three, four, three in one round, a loop over sets that ends unevenly
+    (7, 2048, 3, False, 0), (2048, 2048, 8, False, 1), (2050, 2048, 5, True, 0),
+    (4098, 2048, 4, True, 2), (8190, 2048, 7, True, 0), (8200, 2048, 3, True, 0),
+    (12306, 2048, 6, True, 2), (9, 3072, 8, True, 0), (4104, 3072, 6, False, 1),
+    (6150, 3072, 3, True, 2), (8194, 3072, 5, True, 0), (16402, 3072, 8, True, 2),
+    (2050, 6144, 8, False, 1), (2056, 8192, 5, False, 0), (2040, 8192, 8, False, 1),
+])
+def test_gemv_batched_tiles(torch, yuear_lib, oracle, n, k, batch, norm, epilogue):
+    test_gemv_matches_oracle(torch, yuear_lib, oracle, n, k, batch, norm, epilogue)
+
+
+@pytest.mark.parametrize("k", [2048, 3072])
+def test_gemv_batched_in_place(torch, yuear_lib, oracle, k):
+    # y over x: the workgroups must not read rows that others have written
+    rng = np.random.default_rng(k)
+    w, x, g = bf(rng.normal(size=(k, k)) / k ** 0.5), bf(rng.normal(size=(5, k))), bf(rng.uniform(size=k))
+    dw, dg, dx, dy = (dev(torch, a) for a in (w, g, x, np.zeros_like(x)))
+    for y in (dy, dx):
+        assert yuear_lib.lib.yuear_op_gemv(dw.data_ptr(), k, k, 5, dx.data_ptr(), k, dg.data_ptr(),
+                                           1e-5, y.data_ptr(), k, 0, None) == 0
+    assert_close_bf16(host(torch, dx), host(torch, dy), exact_frac=0.9)
+
+
 @pytest.mark.parametrize("batch", [1, 2, 3, 5, 8])
 def test_gemv_random_shapes_and_strides(torch, yuear_lib, oracle, batch):
     """Seeded sweep per batch size: random N, K (the MFMA form's hidden sizes

@@ -33,13 +33,11 @@ struct GemvParams {
   int epilogue = kEpiStore;
   int seg0_start = 0, seg0_len = 1 << 30, seg1_start = 0;  // row map
   int32_t *advance = nullptr;  // block 0 increments advance[0..batch)
-  // [batch][k] scratch for the batched (MFMA) form: with a gather or an
-  // RMSNorm prologue, a row kernel first writes the prepared rows here once
-  // instead of every workgroup re-normalising them.
+  // optional [batch][k] scratch of the batched (MFMA) form: with it a row kernel
+  // first writes the gathered / normalised rows there (y may then overlap x).
   uint16_t *stage = nullptr;
   // The same weight rows in the MFMA-tiled layout of launch_tile_rows, read
-  // by the batched form when given (1 KiB contiguous per wave-load instead of
-  // 16 row pieces of 64 bytes).
+  // by the batched form when given.
   const uint16_t *w_tiled = nullptr;
   // Affine group-64 quantized weights (bits 8 or 4; 0: bf16 only): codes
   // [rows][k * bits / 32] and one scale | bias << 16 word per group
