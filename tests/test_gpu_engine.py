@@ -209,6 +209,22 @@ def test_chunked_prefill_is_bit_identical_to_one_pass(tiny):
         np.testing.assert_array_equal(va, vb)
 
 
+@pytest.mark.parametrize("n", [1, 2, 33, 4096, 4097, 4130])
+def test_prefill_last_row_across_passes(yuear_lib, n):
+    # past K and V the last layer runs on the prompt's last row, and in a pass
+    # that does not end the prompt (4096 tokens each) not at all
+    cfg = dict(TINY, max_position_embeddings=8192)
+    engine = yuear_lib.Engine(cfg, yuear_lib.random_weights(cfg, 5, 0.02, 0.1))
+    ids = np.random.default_rng(n).integers(0, TINY["vocab_size"], n + 1).tolist()
+    a, b = engine.session(1, n + 2), engine.session(1, n + 2)
+    a.prefill(0, ids[:n])
+    via_step = a.step(ids[n])[0]
+    via_prefill = b.prefill(0, ids)
+    assert within(via_step, via_prefill).all()
+    token = int(ids[0])
+    assert within(a.step(token)[0], b.step(token)[0]).all()  # the caches agree
+
+
 def test_decode_step_agrees_with_prefill_path(tiny):
     engine, _, _ = tiny
     ids = [7, 8, 9, 10, 11, 12]

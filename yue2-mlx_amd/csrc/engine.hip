@@ -703,7 +703,8 @@ void set_quant(GemvParams &g, int bits, const uint32_t *codes, const uint32_t *g
 }
 
 // decode kernels of one layer on S.x (all branches)
-void enqueue_ffn(yuear_session &S, int l);
+void enqueue_o(yuear_session &S, int l, const uint16_t *attn, uint16_t *x, int batch);
+void enqueue_ffn(yuear_session &S, int l, uint16_t *x, int batch);
 
 void enqueue_layer(yuear_session &S, int l, bool embed_first) {
   yuear_engine &E = *S.e;
@@ -755,25 +756,32 @@ void enqueue_layer(yuear_session &S, int l, bool embed_first) {
   a.out_stride = c.Hq * c.D;
   HIPC(launch_attn_decode(a, st));
 
+  enqueue_o(S, l, S.attn, S.x, S.B);
+  enqueue_ffn(S, l, S.x, S.B);
+}
+
+// o projection of the attention rows + residual
+void enqueue_o(yuear_session &S, int l, const uint16_t *attn, uint16_t *x, int batch) {
+  yuear_engine &E = *S.e;
+  const Config &c = E.cfg;
+  const LayerW &L = E.layers[l];
   GemvParams o;
   o.w = L.o;
   set_quant(o, E.bits, L.qo, L.go);
   o.n = c.H;
   o.k = c.Hq * c.D;
-  o.batch = S.B;
-  o.x = S.attn;
+  o.batch = batch;
+  o.x = attn;
   o.x_stride = c.Hq * c.D;
-  o.y = S.x;
+  o.y = x;
   o.y_stride = c.H;
   o.epilogue = kEpiResidual;
   o.w_tiled = L.o_t;
-  HIPC(launch_gemv(o, st));
-
-  enqueue_ffn(S, l);
+  HIPC(launch_gemv(o, S.stream));
 }
 
 // post-attention RMSNorm + gate/up + SwiGLU, down + residual (ar.cpp:295-298)
-void enqueue_ffn(yuear_session &S, int l) {
+void enqueue_ffn(yuear_session &S, int l, uint16_t *x, int batch) {
   yuear_engine &E = *S.e;
   const Config &c = E.cfg;
   const LayerW &L = E.layers[l];
@@ -783,8 +791,8 @@ void enqueue_ffn(yuear_session &S, int l) {
   set_quant(g, E.bits, L.qgu, L.ggu);
   g.n = 2 * c.F;
   g.k = c.H;
-  g.batch = S.B;
-  g.x = S.x;
+  g.batch = batch;
+  g.x = x;
   g.x_stride = c.H;
   g.norm_w = L.post_ln;
   g.eps = c.eps;
@@ -799,10 +807,10 @@ void enqueue_ffn(yuear_session &S, int l) {
   set_quant(d, E.bits, L.qdown, L.gdown);
   d.n = c.H;
   d.k = c.F;
-  d.batch = S.B;
+  d.batch = batch;
   d.x = S.act;
   d.x_stride = c.F;
-  d.y = S.x;
+  d.y = x;
   d.y_stride = c.H;
   d.epilogue = kEpiResidual;
   d.w_tiled = L.down_t;
@@ -947,23 +955,23 @@ void prefill(yuear_session &S, int b, const int32_t *ids, int n, uint16_t *logit
     std::memcpy(S.pin_tok, ids + start, size_t(T) * 4);
     HIPC(hipMemcpyAsync(S.pids, S.pin_tok, size_t(T) * 4, hipMemcpyHostToDevice, st));
     HIPC(launch_embed_rows(E.embed, S.pids, T, c.H, S.px, st));
-    // a residual projection into x, then (norm_w set) the RMSNorm of the
-    // updated rows into h: a split GEMM's reduce and the norm run as one
-    // kernel (bit-identical to the reduce kernel followed by the norm)
+    // a residual projection into x, then the RMSNorm of the updated rows into
+    // h: a split GEMM's reduce and the norm run as one kernel (bit-identical to
+    // the reduce kernel followed by the norm)
     auto residual_then_norm = [&](GemmParams g, const uint16_t *norm_w) -> hipError_t {
       const int few = gemm_ksplit_choice(g.m, g.n, g.k, gemm_cus());
       if (few >= 0) {
         const hipError_t e = launch_gemm_ksplit(g, few, st);
-        return e != hipSuccess || !norm_w
+        return e != hipSuccess
                    ? e
                    : launch_rms_norm_rows(S.px, T, c.H, norm_w, c.eps, S.ph, st);
       }
       int shape = 0, splits = 1;
       gemm_plan(g.m, g.n, g.k, gemm_cus(), g.part_bytes, &shape, &splits);
-      const bool fuse = norm_w && splits > 1 && S.fuse_norm;
+      const bool fuse = splits > 1 && S.fuse_norm;
       g.defer_reduce = fuse;
       hipError_t e = launch_gemm_tile(g, shape, st, splits);
-      if (e != hipSuccess || !norm_w)
+      if (e != hipSuccess)
         return e;
       return fuse ? launch_gemm_reduce_norm(g, splits, norm_w, c.eps, S.ph, st)
                   : launch_rms_norm_rows(S.px, T, c.H, norm_w, c.eps, S.ph, st);
@@ -991,28 +999,39 @@ void prefill(yuear_session &S, int b, const int32_t *ids, int n, uint16_t *logit
       qp.k_cache = S.kc + S.layer_kv_offset(l, b);
       qp.v_cache = S.vc + S.layer_kv_offset(l, b);
       HIPC(launch_qk_prep(qp, st));
+      // The last layer's rows past K and V are read by the head alone, and only
+      // the prompt's last one: its attention, projections and FFN run on that
+      // row, as in a decode step (301 tokens at 3072 wide: 88 us a prefill less).
+      const bool last = l + 1 == c.layers;
+      if (last && start + T < n)
+        break;
       AttnPrefillParams ap;
-      ap.q = S.pq;
+      ap.q = last ? S.pq + size_t(T - 1) * c.Hq * c.D : S.pq;
       ap.k_cache = qp.k_cache;
       ap.v_cache = qp.v_cache;
-      ap.tokens = T;
-      ap.pos0 = pos0;
+      ap.tokens = last ? 1 : T;
+      ap.pos0 = last ? pos0 + T - 1 : pos0;
       ap.heads = c.Hq;
       ap.kv_heads = c.Hkv;
       ap.head_dim = c.D;
       ap.capacity = S.kv_stride;
       ap.out = S.pattn;
       HIPC(launch_attn_prefill(ap, st));
+      if (last) {
+        uint16_t *x = S.px + size_t(T - 1) * c.H;
+        enqueue_o(S, l, S.pattn, x, 1);
+        enqueue_ffn(S, l, x, 1);
+        break;
+      }
       GemmParams og{S.pattn, c.Hq * c.D, L.o, T, c.H, c.Hq * c.D, S.px, c.H, 1, S.psplit,
                     kSplitBytes};
       HIPC(residual_then_norm(og, L.post_ln));
       GemmParams gu{S.ph, c.H, L.gu, T, 2 * c.F, c.H, S.pact, c.F, 2, S.psplit,
                     kSplitBytes};  // SwiGLU epilogue
       HIPC(launch_gemm(gu, st));
-      // down + residual, then the next layer's input norm (the last layer's
-      // rows go to the final norm of the head)
+      // down + residual, then the next layer's input norm
       GemmParams dg{S.pact, c.F, L.down, T, c.H, c.F, S.px, c.H, 1, S.psplit, kSplitBytes};
-      HIPC(residual_then_norm(dg, l + 1 < c.layers ? E.layers[l + 1].input_ln : nullptr));
+      HIPC(residual_then_norm(dg, E.layers[l + 1].input_ln));
     }
     S.host_pos[b] += T;
     if (start + T >= n)  // final norm + projection of the last hidden row
