@@ -209,6 +209,26 @@ def test_chunked_prefill_is_bit_identical_to_one_pass(tiny):
         np.testing.assert_array_equal(va, vb)
 
 
+@pytest.mark.parametrize("branches,vocab", [(1, 9), (3, 509), (8, 2056), (2, 4104)])
+def test_tokens_positions_and_logits_of_every_branch(yuear_lib, branches, vocab):
+    # token and position words of all branches in, logits rows (padded to 16
+    # bytes) out: each branch as a session of its own, after a moved position
+    cfg = dict(TINY, vocab_size=vocab)
+    engine = yuear_lib.Engine(cfg, yuear_lib.random_weights(cfg, 9, 0.02, 0.1))
+    ids = np.random.default_rng(vocab).integers(0, vocab, (branches, 9))
+    s = engine.session(branches, 16)
+    for b in range(branches):
+        s.prefill(b, ids[b, :7].tolist())
+        s.set_position(b, 3 + b % 4)
+    got = [s.step(ids[:, 7 + k].tolist()) for k in range(2)]
+    for b in range(branches):
+        one = engine.session(1, 16)
+        one.prefill(0, ids[b, :3 + b % 4].tolist())
+        for k in range(2):
+            assert within(got[k][b], one.step(int(ids[b, 7 + k]))[0]).all(), (b, k)
+        assert s.position(b) == one.position(0)
+
+
 @pytest.mark.parametrize("n", [1, 2, 33, 4096, 4097, 4130])
 def test_prefill_last_row_across_passes(yuear_lib, n):
     # past K and V the last layer runs on the prompt's last row, and in a pass

@@ -685,12 +685,21 @@ void begin_session(yuear_session &S, yuear_engine *E, int branches, int capacity
   HIPC(hipStreamSynchronize(S.stream));
 }
 
-void set_device_pos(yuear_session &S) {
-  for (int b = 0; b < S.B; ++b)
-    S.pin_tok[b] = S.host_pos[b];
-  HIPC(hipMemcpyAsync(S.pos, S.pin_tok, S.B * 4, hipMemcpyHostToDevice, S.stream));
-  HIPC(hipStreamSynchronize(S.stream));
+// Small host values go to the device as kernel arguments and logits come back
+// through a kernel's stores to pinned memory: both are one launch that neither
+// waits for the stream nor goes through the copy path (whose calls cost the host
+// 5-10 us each, with the GPU idle before a step and after a prefill).
+void put_words(yuear_session &S, int32_t *dst, const int32_t *src) {
+  Words w;
+  std::copy(src, src + S.B, w.v);
+  HIPC(launch_put_words(dst, w, S.B, S.stream));
 }
+void get_logits(yuear_session &S, int b, int rows) {  // into pin_logits from row 0
+  const size_t ls = S.phase.stride();
+  HIPC(launch_copy_out(S.pin_logits, S.logits + size_t(b) * ls, size_t(rows) * ls, S.stream));
+}
+
+void set_device_pos(yuear_session &S) { put_words(S, S.pos, S.host_pos.data()); }
 
 // Quantized codes of a projection: the 1-2 branch GEMVs read them instead
 // of the dequantized rows in `w`.
@@ -1037,15 +1046,15 @@ void prefill(yuear_session &S, int b, const int32_t *ids, int n, uint16_t *logit
     if (start + T >= n)  // final norm + projection of the last hidden row
       enqueue_head(S, S.px + size_t(T - 1) * c.H, 1, c.H,
                    S.logits + size_t(b) * S.phase.stride(), nullptr);
-    HIPC(hipStreamSynchronize(st));
+    else  // pin_tok is read until here
+      HIPC(hipStreamSynchronize(st));
   }
   set_device_pos(S);
-  if (logits_out) {
-    HIPC(hipMemcpyAsync(S.pin_logits, S.logits + size_t(b) * S.phase.stride(),
-                        size_t(S.phase.size) * 2, hipMemcpyDeviceToHost, st));
-    HIPC(hipStreamSynchronize(st));
+  if (logits_out)
+    get_logits(S, b, 1);
+  HIPC(hipStreamSynchronize(st));
+  if (logits_out)
     std::memcpy(logits_out, S.pin_logits, size_t(S.phase.size) * 2);
-  }
 }
 
 void step(yuear_session &S, const int32_t *tokens, uint16_t *logits_out) {
@@ -1059,15 +1068,13 @@ void step(yuear_session &S, const int32_t *tokens, uint16_t *logits_out) {
       invalid("Requested generation budget is exhausted");
   }
   ensure_step_graph(S);
-  std::memcpy(S.pin_tok, tokens, size_t(S.B) * 4);
-  HIPC(hipMemcpyAsync(S.tok, S.pin_tok, size_t(S.B) * 4, hipMemcpyHostToDevice, S.stream));
+  put_words(S, S.tok, tokens);
   HIPC(hipGraphLaunch(S.step_exec, S.stream));
   for (int b = 0; b < S.B; ++b)
     S.host_pos[b] += 1;
   if (logits_out) {
     const size_t ls = S.phase.stride(), n = S.phase.size;
-    HIPC(hipMemcpyAsync(S.pin_logits, S.logits, size_t(S.B) * ls * 2, hipMemcpyDeviceToHost,
-                        S.stream));
+    get_logits(S, 0, S.B);
     HIPC(hipStreamSynchronize(S.stream));
     for (int b = 0; b < S.B; ++b)
       std::memcpy(logits_out + b * n, S.pin_logits + b * ls, n * 2);

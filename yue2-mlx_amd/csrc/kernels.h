@@ -205,6 +205,13 @@ hipError_t launch_gemm_reduce_norm(const GemmParams &p, int splits, const uint16
                                    float eps, uint16_t *y, hipStream_t s);
 void gemm_plan(int m, int n, int k, int cus, size_t part_bytes, int *shape, int *splits);
 
+// dst[0..n) = w.v[0..n), n <= 8; elems bf16 (a multiple of 8) of `src` to
+// pinned host memory.
+struct Words {
+  int32_t v[8];
+};
+hipError_t launch_put_words(int32_t *dst, const Words &w, int n, hipStream_t s);
+hipError_t launch_copy_out(uint16_t *dst, const uint16_t *src, size_t elems, hipStream_t s);
 hipError_t launch_embed_rows(const uint16_t *table, const int32_t *ids, int rows,
                              int width, uint16_t *out, hipStream_t s);
 hipError_t launch_rms_norm_rows(const uint16_t *x, int rows, int width,

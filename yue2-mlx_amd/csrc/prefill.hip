@@ -244,7 +244,34 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill64_kernel(AttnPrefil
   attn::attn_query_tile64<false>(prefill_tile<64>(p), qscale, sh);
 }
 
+__global__ void put_words_kernel(int32_t *dst, Words w, int n) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (int(threadIdx.x) == i && i < n)
+      dst[i] = w.v[i];
+}
+__global__ __launch_bounds__(256) void copy_out_kernel(u32x4 *dst, const u32x4 *src, size_t chunks) {
+  const size_t c = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (c < chunks)
+    dst[c] = src[c];
+}
+
 }  // namespace
+
+hipError_t launch_put_words(int32_t *dst, const Words &w, int n, hipStream_t s) {
+  if (n < 1 || n > 8)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(put_words_kernel, dim3(1), dim3(64), 0, s, dst, w, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_out(uint16_t *dst, const uint16_t *src, size_t elems, hipStream_t s) {
+  if (elems < 8 || elems % 8)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(copy_out_kernel, dim3(unsigned((elems / 8 + 255) / 256)), dim3(256), 0, s,
+                     reinterpret_cast<u32x4 *>(dst), reinterpret_cast<const u32x4 *>(src), elems / 8);
+  return hipGetLastError();
+}
 
 hipError_t launch_embed_rows(const uint16_t *table, const int32_t *ids, int rows, int width,
                              uint16_t *out, hipStream_t s) {
