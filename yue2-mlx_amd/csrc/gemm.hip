@@ -460,15 +460,25 @@ YUEAR_GEMM_KERNEL(gemm_128x128, gemm_tile, 128, 128, 2, 2)
 YUEAR_GEMM_KERNEL(gemm_192x192, gemm_tile16, 192, 192, 2, 4)
 #undef YUEAR_GEMM_KERNEL
 
-// Time model of the tile shapes, in microseconds per 48 K steps measured on
-// MI355X (K = 3072, 256 CUs): `alone` for a tile with a CU to itself on an
-// otherwise idle chip, `busy` with every CU holding one such tile, `round` for
-// a full round of per_cu workgroups on every CU.
+// Time model of the tile shapes, in microseconds per 48 K steps on MI355X (K =
+// 3072, 256 CUs): `alone` for a tile with a CU to itself on an otherwise idle
+// chip, `busy` with every CU holding one such tile, `round` for a full round of
+// per_cu workgroups on every CU. kShapes: fitted to all six shapes on eight
+// projections (2048-16384 rows, K 2048-8192) at 17 token counts from 140 to 3000,
+// weights from HBM; its pick takes 0.14% more than the fastest shape on average
+// (4% at worst; kWarmShapes, fitted with the weights in cache, 1.9% and 18%: 301
+// x 16384 x 3072 65 us against 57, 2500 x 16384 x 3072 253 against 224).
+// kWarmShapes weighs splits of K (gemm_plan), with whose costs it was fitted.
 struct TileShape {
   int bm, bn, per_cu;
   double alone, busy, round;
 };
 constexpr TileShape kShapes[] = {
+    {256, 256, 1, 65.7, 86.7, 83.5}, {256, 128, 1, 47.2, 58.8, 53.7},
+    {128, 256, 1, 41.3, 68.9, 60.9}, {256, 192, 1, 57.7, 72.0, 70.1},
+    {128, 128, 2, 38.5, 46.5, 53.6}, {192, 192, 1, 49.6, 61.3, 59.9},
+};
+constexpr TileShape kWarmShapes[] = {
     {256, 256, 1, 63.0, 85.0, 85.0}, {256, 128, 1, 43.5, 50.0, 50.0},
     {128, 256, 1, 44.3, 50.0, 50.0}, {256, 192, 1, 49.0, 58.0, 58.0},
     {128, 128, 2, 34.3, 40.0, 50.8}, {192, 192, 1, 41.0, 49.0, 49.0},
@@ -687,12 +697,13 @@ int gemm_tile_choice(int m, int n, int cus) {
 // tokens on MI355X: the pick is within 9% of the fastest measured (split or
 // not) in all 28 cases; without a split it is gemm_tile_choice's shape.
 void gemm_plan(int m, int n, int k, int cus, size_t part_bytes, int *shape, int *splits) {
-  *shape = gemm_tile_choice(m, n, cus);
+  const int whole = gemm_tile_choice(m, n, cus);
+  *shape = whole;
   *splits = 1;
   double best_t = 0;
   const double mn = double(m) * double(n);
   for (int i = 0; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
-    const TileShape &t = kShapes[i];
+    const TileShape &t = kWarmShapes[i];
     const long long tiles = (long long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
     const long long slots = (long long)cus * t.per_cu;
     for (int z = 1; z <= kMaxSplits; ++z) {
@@ -710,7 +721,7 @@ void gemm_plan(int m, int n, int k, int cus, size_t part_bytes, int *shape, int 
       if (z > 1)
         time += 4.0 + 0.4e-6 * (4.0 * z * mn + 2.0 * mn) + 0.1e-6 * 4.0 * z * mn;
       if ((i == 0 && z == 1) || time < best_t * 0.999) {
-        *shape = i;
+        *shape = z > 1 ? i : whole;
         *splits = z;
         best_t = time;
       }
