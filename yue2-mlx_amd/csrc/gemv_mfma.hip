@@ -230,8 +230,10 @@ __global__ __launch_bounds__(KW * T * 64) void gemv_mfma_kernel(GemvParams p) {
         xr[i] = u32x4{o[0], o[1], o[2], o[3]};
       }
   }
-  // row b starts at chunk b NCH + b % 4 + 8 (b / 4): the 16 lanes (row, half)
-  // of an operand read then hit 16 different 16-byte slots of the 64 banks
+  // row b starts at chunk b NCH + b % 4 + 8 (b / 4): of the 16 lanes an operand
+  // read is served in at a time, at most two pairs share a 16-byte slot of the 64
+  // banks. (Rows two chunks apart, without conflicts: the same to 0.1 us, but k
+  // 8192, at its register limit, 11.8 -> 13.0 us.)
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     const int b = grp + G * i;
