@@ -640,3 +640,52 @@ def test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, hea
 ])
 def test_attention_prefill_tile_forms(torch, yuear_lib, oracle, T, pos0, heads, kv_heads):
     test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, heads, kv_heads)
+
+
+def one_hot_scores(rng, heads, kv_heads, nq, nk, mag, seen):
+    """q, k of magnitude `mag` whose largest visible score of each query leads by
+    more than fp32 sums of their products can be off, v, and the output: V of
+    that key. seen(t): keys that query t sees."""
+    q = bf(rng.normal(size=(heads, nq, 128)) * mag)
+    k = bf(rng.normal(size=(kv_heads, nk, 128)) * mag)
+    v = bf(rng.normal(size=(kv_heads, nk, 128)))
+    out = np.zeros((heads, nq, 128), np.uint16)
+    per = heads // kv_heads
+    for h in range(heads):
+        kf = f(k[h // per]).astype(np.float64)
+        for t in range(nq):
+            n = seen(t)
+            x = f(q[h, t]).astype(np.float64)
+            if n > 1:  # move the query towards its best key until it leads
+                best = int((kf[:n] @ x).argmax())
+                x = x + kf[best]
+                q[h, t] = bf(x)
+                x = f(q[h, t]).astype(np.float64)
+            sc = kf[:n] @ x
+            top = np.sort(sc)[-2:]
+            # 128 products: each sum's error is below 128 * 2^-24 * sum |products|
+            assert n == 1 or top[1] - top[0] > 2.0 ** -16 * (np.abs(kf[:n]) @ np.abs(x)).max()
+            assert n == 1 or (top[1] - top[0]) * 128 ** -0.5 * 1.44 > 200
+            out[h, t] = v[h // per, sc.argmax()]
+    return q, k, v, out
+
+
+@pytest.mark.parametrize("mag", [1e3, 5e4, 1e6, 1e9])
+@pytest.mark.parametrize("T,pos0,heads,kv_heads", [
+    (3, 37, 2, 1), (17, 700, 2, 1), (40, 200, 24, 8), (33, 1900, 16, 16),  # key-split tiles
+    (130, 0, 96, 1),                                                        # 64-query tile
+])
+def test_attention_prefill_large_scores(torch, yuear_lib, mag, T, pos0, heads, kv_heads):
+    """Scores of 1e8 to 1e20: each query's weight is all on its best key. The
+    exponent of the best key is exactly 0 (score minus maximum, then the scale);
+    a scaled maximum subtracted inside an fma left the rounding error of the
+    product there, and past 2^32 rows came out as inf / inf or 0 / 0."""
+    rng = np.random.default_rng(int(mag) + T)
+    cap = yuear_lib.kv_slots(pos0 + T)
+    q, k, v, want = one_hot_scores(rng, heads, kv_heads, T, cap, mag, lambda t: pos0 + t + 1)
+    a = [dev(torch, x) for x in (q.transpose(1, 0, 2), k, yuear_lib.v_blocked(v))]
+    out = dev(torch, np.zeros((T, heads, 128), np.uint16))
+    assert yuear_lib.lib.yuear_op_attention_prefill(a[0].data_ptr(), a[1].data_ptr(),
+                                                    a[2].data_ptr(), T, pos0, heads, kv_heads, cap,
+                                                    out.data_ptr(), None) == 0
+    np.testing.assert_array_equal(host(torch, out).transpose(1, 0, 2), want)

@@ -80,6 +80,20 @@ def test_nar_attention_tile_forms(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, 
     test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal)
 
 
+@pytest.mark.parametrize("mag", [5e4, 1e9])
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lk,causal", [
+    (2, 1, 9, 70, False), (2, 2, 3, 3000, False),      # whole and dealt key-split tiles
+    (96, 1, 257, 31, False), (96, 8, 65, 65, True),     # 64-query tiles
+])
+def test_nar_attention_large_scores(torch, yuear_lib, mag, Hq, Hkv, Lq, Lk, causal):
+    # every query's weight is all on one key (see test_attention_prefill_large_scores)
+    from test_gpu_kernels import one_hot_scores
+    rng = np.random.default_rng(int(mag) + Lk)
+    q, k, v, want = one_hot_scores(rng, Hq, Hkv, Lq, Lk, mag, lambda t: t + 1 if causal else Lk)
+    got = yuear_lib.nar_attention(*(dev(torch, x[None]) for x in (q, k, v)), causal)
+    np.testing.assert_array_equal(host(torch, got)[0], want)
+
+
 def test_nar_attention_zero_pads_the_last_key_block(torch, yuear_lib, oracle):
     # 50 keys leave 14 padding slots in the last 32-key block of the
     # workspace: a workspace full of NaN must not reach the output

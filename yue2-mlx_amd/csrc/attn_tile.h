@@ -38,20 +38,22 @@ struct QueryTile {
   size_t out_stride = 0;
   // key-split tile, non-causal: key blocks [blk0, blk1) of the tile (blk1 0:
   // all) and, when set, an unnormalised partial per query instead of out: 132
-  // floats {o[128], m, l, pad} at part + query * 132 (m the running maximum in
-  // the exp2 domain, l the sum of exp2(s - m), o the sum of exp2(s - m) v)
+  // floats {o[128], m, l, pad} at part + query * 132 (m the largest raw score,
+  // l the sum of exp2((s - m) qscale), o that of exp2((s - m) qscale) v)
   int blk0 = 0, blk1 = 0;
   float *part = nullptr;
 };
 
 // One online-softmax step of a lane's query over 8 N / 2 raw scores st (16-key
 // rows of S^T, masked to -inf where not visible): updates the running maximum
-// m (of score * qscale) and this lane's part l of the denominator, leaves the
-// three truncated bf16 pieces of p = exp2(score * qscale - m) in pw per 32
+// m (of the raw scores) and this lane's part l of the denominator, leaves the
+// three truncated bf16 pieces of p = exp2((score - m) * qscale) in pw per 32
 // keys (the top 8, next 8 and last 8 significant bits of p; each remainder is
 // exact, so p is their sum), and returns the factor for the previous O. The
-// scale is applied in the exponent's fma: one rounding less than a scaled
-// score, and one instruction.
+// difference is taken first, so the largest score's exponent is exactly 0
+// whatever its size (fma(score, qscale, -round(m * qscale)) leaves it the
+// rounding error of the product: past 2^32 that overflows exp2 or underflows
+// every weight).
 template <int N>
 __device__ __forceinline__ float softmax_step(const f32x4 (&st)[N], float qscale, float &m_run,
                                               float &l_run, uint32_t (&pw)[N / 2][3][4]) {
@@ -59,18 +61,18 @@ __device__ __forceinline__ float softmax_step(const f32x4 (&st)[N], float qscale
 #pragma unroll
   for (int e = 1; e < 4 * N; ++e)
     mx = fmaxf(mx, st[e >> 2][e & 3]);
-  mx = max_halves(max_row_pairs(mx)) * qscale;
+  mx = max_halves(max_row_pairs(mx));
   const float m_new = fmaxf(m_run, mx);
   const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
-  const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
+  const float corr = __builtin_amdgcn_exp2f((m_run - m_use) * qscale);
   float ps = 0.f;
 #pragma unroll
   for (int g = 0; g < N / 2; ++g)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const f32x4 &s = st[2 * g + (q >> 1)];
-      float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * (q & 1)], qscale, -m_use));
-      float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * (q & 1) + 1], qscale, -m_use));
+      float p0 = __builtin_amdgcn_exp2f((s[2 * (q & 1)] - m_use) * qscale);
+      float p1 = __builtin_amdgcn_exp2f((s[2 * (q & 1) + 1] - m_use) * qscale);
       ps += p0;
       ps += p1;
 #pragma unroll
@@ -297,7 +299,7 @@ __device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale
 #pragma unroll
   for (int w = 0; w < W; ++w) {
     const float m = sh.m[w][c][i];
-    f[w] = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    f[w] = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((m - M) * qscale);
     L += f[w] * sh.l[w][c][i];
   }
   const int qi = 16 * c + i;

@@ -104,14 +104,14 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void nar_attn64_kernel(NarAttnParams 
   attn::attn_query_tile64<true>(nar_tile<64>(p, blockIdx.x, tile), qscale, sh);
 }
 
-// out[row][d] = bf16(sum_s w_s o_s[d] / sum_s w_s l_s), w_s = exp2(m_s - max m)
+// out[row][d] = bf16(sum_s w_s o_s[d] / sum_s w_s l_s), w_s = exp2((m_s - max m) qscale)
 // over the up to kPieces partials of each query row of a tile that more than
 // one workgroup holds; one thread per (row, 4 dims). All of a thread's loads
 // are issued before the first use (a piece it lacks is read as its last one,
 // with weight 0).
 template <int kPieces>
-__global__ __launch_bounds__(256) void nar_merge_kernel(NarAttnParams p, int kq, int steps,
-                                                        int per_head, int total) {
+__global__ __launch_bounds__(256) void nar_merge_kernel(NarAttnParams p, float qscale, int kq,
+                                                        int steps, int per_head, int total) {
   const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
   const int row = int(idx / 32);
   if (row >= p.batch * p.heads * p.q_len)
@@ -143,7 +143,9 @@ __global__ __launch_bounds__(256) void nar_merge_kernel(NarAttnParams p, int kq,
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < kPieces; ++s) {
-    const float w = s > n || ml[s].x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ml[s].x - M);
+    const float w = s > n || ml[s].x == -__builtin_inff()
+                        ? 0.f
+                        : __builtin_amdgcn_exp2f((ml[s].x - M) * qscale);
     L += w * ml[s].y;
     o += w * v[s];
   }
@@ -233,7 +235,8 @@ hipError_t launch_nar_attention(NarAttnParams p, hipStream_t s) {
                : pieces <= 4 ? nar_merge_kernel<4>
                : pieces <= 8 ? nar_merge_kernel<8>
                              : nar_merge_kernel<attn::kMaxPieces>;
-  hipLaunchKernelGGL(merge, mgrid, dim3(256), 0, s, p, plan.queries, steps, per_head, total);
+  hipLaunchKernelGGL(merge, mgrid, dim3(256), 0, s, p, qscale, plan.queries, steps, per_head,
+                     total);
   return hipGetLastError();
 }
 
