@@ -637,6 +637,9 @@ def test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, hea
     # 64-query tiles with an odd last block (tail step) and a ragged last tile
     (1, 0, 1, 1), (16, 240, 8, 8), (17, 240, 6, 2), (160, 97, 24, 8), (33, 2000, 24, 8),
     (301, 607, 24, 8), (341, 0, 24, 8), (700, 0, 24, 8), (681, 1969, 24, 8),
+    # 64-query tiles one block a step, by 16 heads a last tile of one query;
+    # two blocks a step; 32 queries by 8 waves
+    (513, 0, 96, 16), (341, 420, 96, 32), (257, 32, 48, 16), (700, 2301, 6, 2),
 ])
 def test_attention_prefill_tile_forms(torch, yuear_lib, oracle, T, pos0, heads, kv_heads):
     test_attention_prefill_matches_oracle(torch, yuear_lib, oracle, T, pos0, heads, kv_heads)

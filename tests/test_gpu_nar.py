@@ -67,14 +67,22 @@ def test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, 
     # whole key-split tiles of 16 and 32 queries, 4 and 8 waves: fewer blocks
     # than waves, a partial last block, a last tile of one query
     (1, 1, 1, 1, 31, False), (2, 6, 3, 17, 289, False), (1, 1, 1, 1, 697, False),
-    (1, 24, 8, 651, 31, False), (1, 6, 3, 677, 919, False),
-    # dealt: 9, 9, 8 and 13 pieces a tile at most, a ragged last tile, steps
-    # and blocks that do not divide
+    (1, 6, 3, 677, 919, False), (1, 24, 8, 300, 1100, False), (1, 24, 8, 250, 3600, False),
+    (1, 24, 8, 1001, 1500, False),
+    # dealt to all CUs: key-split tiles of 16 and 32 queries by 8 waves, steps
+    # and blocks that do not divide, a ragged last tile
     (2, 16, 8, 1, 4001, False), (1, 16, 8, 53, 2000, False), (1, 24, 8, 53, 6500, False),
-    (1, 6, 3, 274, 6000, False), (1, 16, 8, 100, 8001, False), (1, 24, 8, 250, 3600, False),
-    # 64-query tiles, an odd last block; causal forms
-    (1, 12, 4, 677, 31, False), (1, 24, 8, 1024, 400, False), (1, 24, 8, 100, 100, True),
-    (1, 24, 8, 449, 449, True), (1, 48, 16, 850, 850, True),
+    (1, 6, 3, 274, 6000, False), (1, 16, 8, 100, 8001, False),
+    # ... to fewer workgroups, as few keys or heads allow: 8, 56, 72, 104, 208
+    (1, 1, 1, 1, 20000, False), (1, 1, 1, 100, 2000, False), (1, 2, 1, 33, 8001, False),
+    (1, 2, 2, 130, 1500, False), (1, 16, 8, 17, 12001, False), (1, 1, 1, 65, 1500, False),
+    # ... 4 waves, 264 and 360 workgroups; 64-query tiles, an odd last block
+    (1, 1, 1, 341, 3001, False), (1, 6, 2, 65, 3001, False), (1, 24, 8, 341, 1500, False),
+    (1, 2, 1, 341, 6001, False),
+    # 64-query tiles, one and two blocks a step, an odd last block; causal forms
+    (1, 12, 4, 677, 31, False), (1, 24, 8, 1024, 400, False), (1, 48, 16, 1025, 97, False),
+    (1, 24, 8, 1001, 289, False), (1, 24, 8, 100, 100, True),
+    (1, 24, 8, 449, 449, True), (1, 48, 16, 850, 850, True), (2, 48, 16, 330, 330, True),
 ])
 def test_nar_attention_tile_forms(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal):
     test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal)

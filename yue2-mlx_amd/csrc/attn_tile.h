@@ -12,9 +12,9 @@
 // or 8 waves split the tile's 32-key blocks and merges their (m, l, O) through
 // LDS: for launches with few tiles, whose time is the longest wave's chain of
 // blocks and the rate at which one CU pulls K and V (4 waves: two workgroups
-// to a CU, for more tiles than CUs). The 64-query tile
-// (attn_query_tile64) has its 4 waves walk the same blocks, fetched once per
-// workgroup: for launches that fill the GPU, bound by VALU and MFMA issue.
+// to a CU, for more tiles than CUs). The 64-query tile (attn_query_tile64) has
+// its 4 waves walk the same blocks, fetched once per workgroup, one or two a
+// step: for launches that fill the GPU, bound by VALU and MFMA issue.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -327,25 +327,28 @@ __device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale
 
 // ---------------------------------------------------------------------------
 // 64-query tile with K/V shared through LDS: wave w owns queries 16 w + i and
-// all four waves walk the same keys, 64 per step (two 32-key blocks: one
+// all four waves walk the same keys, N 32-key blocks per step (N = 2: one
 // rescale of O and one cross-lane maximum for both). Each block's K and V are
 // fetched once per workgroup (each wave loads a quarter: K pieces and V dim
 // tiles 2 w, 2 w + 1 in the MFMA operand layout of load_k / load_v, which the
 // operand reads then find at constant offsets; whole-KiB loads with swizzled
 // reads measured 0-8% slower here) into an LDS ring of two steps, one step
 // ahead; every wave reads its operands from LDS. No merge across waves.
-struct Tile64Lds {  // 64 KiB: two workgroups per CU, two waves per SIMD
-  u32x4 k[2][2][8][64];  // [stage][32-key block][piece][lane]
-  u32x4 v[2][2][8][64];
+template <int N>
+struct Tile64Lds {  // N = 2: 64 KiB, two workgroups per CU; N = 1: 32 KiB, five
+  u32x4 k[2][N][8][64];  // [stage][32-key block][piece][lane]
+  u32x4 v[2][N][8][64];
 };
+template <int N>
+constexpr int kTile64Waves = N == 1 ? 5 : 2;  // waves per SIMD (LDS, registers)
 
-template <bool kRows>
+template <bool kRows, int N>
 __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qscale,
-                                                  Tile64Lds &sh) {
+                                                  Tile64Lds<N> &sh) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane >> 4, i = lane & 15;
-  const int nblk = (t.kend + kBlock - 1) / kBlock, nkeys = nblk * kBlock;
+  const int nblk = t.blk1 ? t.blk1 : (t.kend + kBlock - 1) / kBlock, nkeys = nblk * kBlock;
   const int last = t.kend - 1;
   u32x4 qb[4];
   {
@@ -357,18 +360,18 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
   }
   const int kmax = t.causal_pos >= 0 ? t.causal_pos + 16 * wave + i : t.kv_len - 1;
   const auto rk = k_rsrc(t), rv = v_rsrc<kRows>(t);
-  // this wave's quarter of the two blocks at kb0 into `stage`: K pieces 2 w,
+  // this wave's quarter of the N blocks at kb0 into `stage`: K pieces 2 w,
   // 2 w + 1 (T = w / 2, s = 2 (w % 2) + {0, 1}) and V dim tiles 2 w, 2 w + 1.
   // Keys are clamped to the last visible one.
   auto fetch = [&](int kb0, int stage) {
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+    for (int g = 0; g < N; ++g) {
       const int kb = kb0 + kBlock * g;
       const int key = min(kb + key_ofs(wave >> 1, i), last);
       const uint32_t ko = uint32_t(key * (D / 8) + 8 * (wave & 1) + r) * 16;
       // the missing half of an odd last step: V past the range, zeros (its
       // weights are zero, and 0 * inf of another block would be NaN)
-      const uint32_t vb = uint32_t(min(kb, nkeys)) * (D * 2);
+      const uint32_t vb = uint32_t(N > 1 ? min(kb, nkeys) : kb) * (D * 2);
       const uint32_t vo0 = vb + (kRows ? v_row_fetch(lane, 2 * wave)
                                        : uint32_t((32 * wave + i) * (kBlock / 8) + r) * 16);
       const uint32_t vo1 = kRows ? vb + v_row_fetch(lane, 2 * wave + 1) : vo0 + 1024;
@@ -388,42 +391,54 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt)
     o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = (nblk + 1) / 2;
-  fetch(0, 0);
+  const int first = t.blk0 / N, steps = (nblk + N - 1) / N;  // steps [first, steps)
+  fetch(N * first * kBlock, first & 1);
   __builtin_amdgcn_s_waitcnt(0);  // (a barrier waits for no load)
   __syncthreads();
-  // one step of 64 keys; kMask: the causal / key-length mask, needed only from
-  // the first step with a key past the smallest kmax of the tile's queries
+  // one step of 32 N keys; kMask: the causal / key-length mask, needed only
+  // from the first step with a key past the smallest kmax of the tile's queries
   auto step = [&](int x, auto mask_tag) {
     constexpr bool kMask = decltype(mask_tag)::value;
-    const int stage = x & 1, kb = 2 * x * kBlock;
+    const int stage = x & 1, kb = N * x * kBlock;
     // step x + 1 into the stage every wave finished reading before the
     // previous barrier; in flight during this step's products
     if (x + 1 < steps)  // uniform
-      fetch(kb + 2 * kBlock, stage ^ 1);
-    // four independent chains of four dependent MFMAs, interleaved
-    f32x4 st[4];
+      fetch(kb + N * kBlock, stage ^ 1);
+    // 2 N independent chains of four dependent MFMAs, interleaved
+    f32x4 st[2 * N];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 2 * N; ++j)
       st[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 2 * N; ++j)
         st[j] = mfma(sh.k[stage][j >> 1][4 * (j & 1) + s][lane], qb[s], st[j]);
     if constexpr (kMask) {  // lane (query 16 w + i, r): keys kb + 32 g + 8 r + 4 T + u
 #pragma unroll
-      for (int e = 0; e < 16; ++e)
+      for (int e = 0; e < 8 * N; ++e)
         if (kb + 32 * (e >> 3) + 8 * r + (e & 7) > kmax)
           st[e >> 2][e & 3] = -__builtin_inff();
     }
-    uint32_t pw[2][3][4];
-    const float corr = softmax_step<4>(st, qscale, m_run, l_run, pw);
+    uint32_t pw[N][3][4];
+    const float corr = softmax_step<2 * N>(st, qscale, m_run, l_run, pw);
+    if constexpr (N == 1) {  // dim tile by dim tile: 96 registers
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-      o[dt] *= corr;
+      for (int dt = 0; dt < 8; ++dt) {
+        const u32x4 vr = kRows ? v_row_operand(sh.v[stage][0][0], v_row_read(lane, dt))
+                               : sh.v[stage][0][dt][lane];
+        o[dt] *= corr;
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
+        for (int k = 0; k < 3; ++k)
+          o[dt] = mfma(vr, piece(pw[0][k]), o[dt]);
+      }
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt)
+        o[dt] *= corr;
+    }
+#pragma unroll
+    for (int g = 0; g < (N == 1 ? 0 : N); ++g) {
       u32x4 vr[8];
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt)
@@ -439,8 +454,8 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
     __syncthreads();
   };
   const int kfull = t.causal_pos >= 0 ? t.causal_pos + 1 : t.kv_len;
-  int x = 0;
-  for (; x < min(kfull / (2 * kBlock), steps); ++x)
+  int x = first;
+  for (; x < min(kfull / (N * kBlock), steps); ++x)
     step(x, std::false_type{});
   for (; x < steps; ++x)
     step(x, std::true_type{});
@@ -449,6 +464,17 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
   const int qi = 16 * wave + i;
   if (qi >= t.nq)
     return;
+  if (t.part) {
+    float *pq = t.part + size_t(qi) * 132;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+      *reinterpret_cast<f32x4 *>(pq + 16 * dt + 4 * r) = o[dt];
+    if (r == 0) {
+      pq[128] = m_run;
+      pq[129] = L;
+    }
+    return;
+  }
   uint16_t *dst = t.out + size_t(qi) * t.out_stride;
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt)
@@ -456,67 +482,99 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
 }
 
 // How a launch of `heads` heads (batch included) x q_len queries over kv_len
-// keys is cut: queries and waves per workgroup (64: attn_query_tile64, else
-// the key-split tile) and, where the keys may be dealt (non-causal, key-split),
-// groups > 0: the steps of all tiles, `waves` key blocks each, go to that many
-// workgroups in equal contiguous runs, merged by another kernel. (64-query
-// tiles dealt gave no more than the 32-query ones: 512 x 3512, 24 heads, 57 and
-// 57 us.)
-//
-// By a time model in us, fitted on MI355X's 256 CUs at 24/8 and 16/8 heads to
-// 90 non-causal shapes (33-1024 queries x 400-8000 keys) and 150 causal ones
-// (9-3000 queries after 0-2000 keys), every form timed: the pick is within
-// 0.8% of the fastest form on average (10% at worst) and takes 0.72 of the
-// time of the forms before (32 queries by 4 waves from registers; 64 queries,
-// ranges of keys for up to 768 workgroups). A round of workgroups costs
-// `launch`; a step costs `alone` where a workgroup has a CU to itself and
-// `shared` (`causal`: tiles of unequal length) where two do, eight waves
-// always; a further tile of a dealt run 0.8; the merge 5.0 and 0.35 per MB of
-// partials.
+// keys is cut: queries and waves per workgroup (64: attn_query_tile64 with
+// `blocks` key blocks a step, else the key-split tile) and, where the keys may
+// be dealt (non-causal), groups > 0: the steps of all tiles go to that many
+// workgroups in equal contiguous runs, merged by another kernel.
 struct TilePlan {
   int queries = 64, waves = 4, groups = 0;
+  int blocks = 2;
+  int step_blocks() const { return queries == 64 ? blocks : waves; }
 };
 constexpr int kMaxPieces = 16;  // workgroups that may hold parts of a dealt tile
+// Workgroups for `total` steps of tiles of `steps` each: a multiple of 8, at
+// most `slots`, with at least two steps a workgroup and at most kMaxPieces
+// pieces a tile (and total * groups in 31 bits, which the kernels count in); 0:
+// no more workgroups than tiles.
+inline int deal_groups(long long total, long long steps, int slots) {
+  const long long per = std::max<long long>(2, (steps - 1) / (kMaxPieces - 1) + 1);
+  const long long g = std::min<long long>(slots, total / per) / 8 * 8;
+  return total < (1 << 21) && g * steps > total ? int(g) : 0;
+}
+// By a time model in us, fitted on MI355X's 256 CUs, every form timed: 1571
+// causal shapes (1-192 heads, 1-12000 queries after 0-20000 keys) and 1704 others
+// (1-192 heads, 1-5000 queries x 20-24000 keys). Of the launches over 9 us the pick
+// is 0.3% / 1.7% from the fastest form on average (12% / 47% at worst: few queries
+// a head over caches past L2, where the order in which workgroups meet the same
+// keys decides). A step of a tile costs `alone` where a workgroup has a CU to
+// itself and `full` where as many as fit do (`slots` on the chip), in between in
+// proportion; a further round of workgroups costs `round`. Causal tiles are of
+// unequal length: the longest one's chain, or `spread` times the mean of all.
+//
+// Which form where: key-split tiles while 64-query tiles leave CUs idle; one
+// round of 64-query tiles two blocks a step; past it, one block a step, five
+// workgroups to a CU, hides more latency and shares K and V in L2 among more
+// tiles (24 heads x 8 x 2500 x 8000: 4.1 ms, dealt key-split tiles, which a model
+// fitted to batch 1 took, 7.1; 64 heads x 4096 causal 540 us, two blocks 563).
+// Key-split tiles past one round only for up to 64 heads: more heads pull K and
+// V past L2 (24 heads x 8 x 160 x 8000: 372 us, 596 key-split). Dealt: few heads
+// and long caches (1 head x 1 x 20000: 99 us undealt, 19 dealt to 8 workgroups).
 inline TilePlan attn_tile_plan(long long heads, int q_len, int kv_len, bool causal, bool deal) {
   struct Form {
-    int queries, waves;
-    double launch, alone, shared, causal;
+    int queries, waves, blocks, slots;
+    double launch, round, alone, full, spread;  // spread: causal
+    double deal = 0, deal_full = 0, merge = 0, merge_mb = 0;  // dealt to <= 256 / more workgroups
   };
-  static const Form forms[] = {{16, 4, 3.3, 0.82, 1.30, 1.24}, {16, 8, 4.3, 1.18, 1.18, 1.31},
-                               {32, 4, 4.4, 1.13, 1.99, 1.52}, {32, 8, 5.3, 1.98, 1.98, 1.96},
-                               {64, 4, 4.4, 1.20, 2.02, 1.24}};
+  static const Form whole[] = {
+      {16, 4, 0, 512, 4.468, 1.41, 0.9603, 1.568, 0, 0.8873, 1.623, 1.925, 0.5537},
+      {16, 8, 0, 256, 4.574, 8.894, 1.106, 5.091, 0, 1.692, 0, 2.057, 0.177},
+      {32, 4, 0, 512, 5.886, 1.447, 1.113, 2.081, 0, 0.8195, 5.109, 2.233, 0.5655},
+      {32, 8, 0, 256, 7.677, 35.84, 1.647, 1.84, 0, 2.142, 0, 3.061, 0.2742},
+      {64, 4, 2, 512, 5.386, 27.74, 1.122, 1.901, 0, 2, 1.614, 1.833, 0.5814},
+      {64, 4, 1, 1280, 5.319, 0.2201, 0.6365, 2.38, 0}};
+  static const Form tri[] = {
+      {16, 4, 0, 512, 4.499, 8.94, 1.016, 1.214, 1.218},
+      {16, 8, 0, 256, 6.903, 4.535, 0.8857, 1.604, 1.296},
+      {32, 4, 0, 512, 5.473, 12.35, 1.32, 1.823, 1.073},
+      {32, 8, 0, 256, 7.815, 10.35, 2.116, 2.201, 1.103},
+      {64, 4, 2, 512, 4.666, 9.123, 1.19, 1.601, 1.212},
+      {64, 4, 1, 1280, 4.695, 0, 0.6214, 1.485, 1.353}};
   const int nb = (kv_len + kBlock - 1) / kBlock;
   TilePlan best;
   double best_t = __builtin_inf();
   auto take = [&](const Form &f, int groups, double t) {
     if (t < best_t) {
-      best = TilePlan{f.queries, f.waves, groups};
+      best = TilePlan{f.queries, f.waves, groups, f.blocks};
       best_t = t;
     }
   };
-  for (const Form &f : forms) {
-    const int blocks = f.queries == 64 ? 2 : f.waves, slots = f.waves == 8 ? 256 : 512;
+  for (const Form &f : causal ? tri : whole) {
+    const int blocks = f.queries == 64 ? f.blocks : f.waves, per_cu = f.slots / 256;
     const long long tiles = heads * ((q_len + f.queries - 1) / f.queries);
     const long long steps = (nb + blocks - 1) / blocks, total = tiles * steps;
-    const double busy = causal ? f.causal : f.shared, alone = f.waves == 8 ? busy : f.alone;
-    // past three rounds the key-split tiles lose to the 64-query one (3000
-    // queries after 0 keys, 16 heads: 85 against 77 us)
-    if (f.queries == 64 || tiles <= 1536) {
-      const double mean =
-          causal ? (nb - std::max(0, q_len - f.queries) / 64.0) / blocks : double(steps);
-      const long long rem = tiles % slots;
-      const double rate =
-          double(tiles / slots) * busy + (rem == 0 ? 0.0 : rem <= 256 ? alone : busy);
-      take(f, 0, f.launch * double((tiles + slots - 1) / slots) +
-                     std::max((tiles <= 256 ? alone : busy) * double(steps), rate * mean));
+    // a step where n workgroups, less than a full chip, are spread over the CUs
+    auto step = [&](long long n) {
+      return f.alone +
+             (per_cu == 1 ? 0.0 : (f.full - f.alone) * double((n - 1) / 256) / (per_cu - 1));
+    };
+    if (f.queries == 64 || tiles <= (heads <= 64 ? 1536 : 512)) {
+      const long long full = tiles / f.slots, rem = tiles % f.slots;
+      const double rate = double(full) * f.full + (rem ? step(rem) : 0.0);
+      if (causal) {
+        const double mean = (nb - std::max(0, q_len - f.queries) / 64.0) / blocks;
+        take(f, 0, f.launch + f.round * std::max(0.0, double(tiles) / f.slots - 1) +
+                       std::max(step(std::min<long long>(tiles, f.slots)) * double(steps),
+                                f.spread * rate * mean));
+      } else {
+        take(f, 0, f.launch + f.round * double(full + (rem > 0) - 1) + rate * double(steps));
+      }
     }
-    // dealt: at least two steps a workgroup, at most kMaxPieces pieces a tile
-    // (and total * slots in 31 bits, which the kernels count in)
-    if (deal && !causal && f.queries < 64 && total >= 2 * slots && total < (1 << 21) &&
-        (steps - 1) / (total / slots) + 2 <= kMaxPieces) {
-      const double mb = double(slots + std::min<long long>(slots, tiles)) * f.queries * (132 * 4e-6);
-      take(f, slots, f.launch + 0.8 * double(tiles) / slots +
-                         f.shared * double((total + slots - 1) / slots) + 5.0 + 0.35 * mb);
+    const int groups = deal && f.deal > 0 ? deal_groups(total, steps, f.slots) : 0;
+    if (groups) {
+      const double mb = double(groups + std::min<long long>(groups, tiles)) * f.queries * (132 * 4e-6);
+      take(f, groups, f.launch + f.merge + f.merge_mb * mb +
+                          (groups <= 256 ? f.deal : f.deal_full) *
+                              double((total + groups - 1) / groups));
     }
   }
   return best;

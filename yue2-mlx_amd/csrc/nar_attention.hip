@@ -97,11 +97,15 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void nar_attn_kernel(NarAttnParams p,
     __syncthreads();  // the merge has read the stages
   });
 }
+// 64 queries per workgroup, N key blocks a step.
+template <int N>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(2, 2))) void nar_attn64_kernel(NarAttnParams p, float qscale) {
-  __shared__ attn::Tile64Lds sh;
-  const int tile = p.causal ? gridDim.y - 1 - blockIdx.y : blockIdx.y;  // longest first
-  attn::attn_query_tile64<true>(nar_tile<64>(p, blockIdx.x, tile), qscale, sh);
+__attribute__((amdgpu_waves_per_eu(attn::kTile64Waves<N>, attn::kTile64Waves<N>))) void
+nar_attn64_kernel(NarAttnParams p, float qscale) {
+  __shared__ attn::Tile64Lds<N> sh;
+  nar_run<64, N>(p, [&](const attn::QueryTile &t) {
+    attn::attn_query_tile64<true, N>(t, qscale, sh);  // ends with its reads done
+  });
 }
 
 // out[row][d] = bf16(sum_s w_s o_s[d] / sum_s w_s l_s), w_s = exp2((m_s - max m) qscale)
@@ -222,13 +226,16 @@ hipError_t launch_nar_attention(NarAttnParams p, hipStream_t s) {
     hipLaunchKernelGGL((nar_attn_kernel<2, 4>), grid, threads, 0, s, p, qscale);
   else if (plan.queries == 32)
     hipLaunchKernelGGL((nar_attn_kernel<2, 8>), grid, threads, 0, s, p, qscale);
+  else if (plan.blocks == 1)
+    hipLaunchKernelGGL(nar_attn64_kernel<1>, grid, threads, 0, s, p, qscale);
   else
-    hipLaunchKernelGGL(nar_attn64_kernel, grid, threads, 0, s, p, qscale);
+    hipLaunchKernelGGL(nar_attn64_kernel<2>, grid, threads, 0, s, p, qscale);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || !plan.groups)
     return e;
   const int nb = (p.kv_len + kBlock - 1) / kBlock;
-  const int steps = (nb + plan.waves - 1) / plan.waves, total = heads * per_head * steps;
+  const int steps = (nb + plan.step_blocks() - 1) / plan.step_blocks();
+  const int total = heads * per_head * steps;
   const int pieces = (steps - 1) / (total / plan.groups) + 2;  // at most
   const dim3 mgrid(unsigned(((long long)heads * p.q_len * 32 + 255) / 256));
   auto merge = pieces <= 2   ? nar_merge_kernel<2>

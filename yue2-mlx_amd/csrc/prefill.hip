@@ -237,11 +237,12 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(AttnPrefillP
   __shared__ attn::TileLds<C, W> sh;
   attn::attn_query_tile<C, false, W>(prefill_tile<16 * C>(p), qscale, sh);
 }
+template <int N>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill64_kernel(AttnPrefillParams p,
-                                                                      float qscale) {
-  __shared__ attn::Tile64Lds sh;
-  attn::attn_query_tile64<false>(prefill_tile<64>(p), qscale, sh);
+__attribute__((amdgpu_waves_per_eu(attn::kTile64Waves<N>, attn::kTile64Waves<N>))) void
+attn_prefill64_kernel(AttnPrefillParams p, float qscale) {
+  __shared__ attn::Tile64Lds<N> sh;
+  attn::attn_query_tile64<false, N>(prefill_tile<64>(p), qscale, sh);
 }
 
 __global__ void put_words_kernel(int32_t *dst, Words w, int n) {
@@ -316,8 +317,10 @@ hipError_t launch_attn_prefill(const AttnPrefillParams &p, hipStream_t s) {
     hipLaunchKernelGGL((attn_prefill_kernel<2, 4>), grid, threads, 0, s, p, qscale);
   else if (plan.queries == 32)
     hipLaunchKernelGGL((attn_prefill_kernel<2, 8>), grid, threads, 0, s, p, qscale);
+  else if (plan.blocks == 1)
+    hipLaunchKernelGGL(attn_prefill64_kernel<1>, grid, threads, 0, s, p, qscale);
   else
-    hipLaunchKernelGGL(attn_prefill64_kernel, grid, dim3(256), 0, s, p, qscale);
+    hipLaunchKernelGGL(attn_prefill64_kernel<2>, grid, threads, 0, s, p, qscale);
   return hipGetLastError();
 }
 
