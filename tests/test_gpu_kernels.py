@@ -692,3 +692,33 @@ def test_attention_prefill_large_scores(torch, yuear_lib, mag, T, pos0, heads, k
                                                     a[2].data_ptr(), T, pos0, heads, kv_heads, cap,
                                                     out.data_ptr(), None) == 0
     np.testing.assert_array_equal(host(torch, out).transpose(1, 0, 2), want)
+
+
+def test_attention_prefill_past_2_24_keys(torch, yuear_lib):
+    """A cache of more than 2^24 slots (4 GiB of K a head): the key-split tile
+    addresses each block on its own, where one buffer's 32-bit range wraps."""
+    pos0, T = (1 << 24) + 40, 3
+    cap = yuear_lib.kv_slots(pos0 + T)
+    kc = torch.zeros(cap, 128, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros(cap * 128, dtype=torch.bfloat16, device="cuda")
+    rng = np.random.default_rng(2)
+    q = bf(rng.normal(size=(T, 1, 128)))
+    slots = [5, (1 << 24) - 1, 1 << 24, (1 << 24) + 33, pos0 + T - 1]
+    kv = bf(rng.normal(size=(len(slots), 128))), bf(rng.normal(size=(len(slots), 128)))
+    for j, t in enumerate(slots):
+        # scores around 16 of the exp2 domain, so that a slot's weight counts
+        # against the 2^24 slots of score 0
+        kv[0][j] = bf(f(kv[0][j]) * 0.2 + f(q[:, 0]).mean(0) * 3.0)
+        kc[t] = dev(torch, kv[0][j]).view(torch.bfloat16)
+        vc.view(-1, 128, 32)[t // 32, :, t % 32] = dev(torch, kv[1][j]).view(torch.bfloat16)
+    out = dev(torch, np.zeros((T, 128), np.uint16))
+    dq = dev(torch, q)
+    assert yuear_lib.lib.yuear_op_attention_prefill(dq.data_ptr(), kc.data_ptr(), vc.data_ptr(), T,
+                                                    pos0, 1, 1, cap, out.data_ptr(), None) == 0
+    got = f(host(torch, out))
+    for t in range(T):
+        see = [j for j, s in enumerate(slots) if s <= pos0 + t]
+        e = np.exp(f(kv[0][see]).astype(np.float64) @ f(q[t, 0]).astype(np.float64) / 128 ** 0.5)
+        ref = e @ f(kv[1][see]) / (e.sum() + pos0 + t + 1 - len(see))
+        # the sum of 2^24 equal weights in fp32 partial sums of 2^17 each
+        np.testing.assert_allclose(got[t], ref, rtol=2 ** -7, atol=2 ** -8 * np.abs(ref).max())

@@ -100,16 +100,13 @@ __device__ __forceinline__ void store_dims(uint16_t *dst, int d, f32x4 o, float 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
 // Buffers over a tile's K rows and V: reads past the last key (of V in blocks:
-// past its last block) give zeros; the scores of those keys are masked.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t k_rsrc(const QueryTile &t) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(t.kc), 0, uint32_t(t.kend) * (D * 2),
-                                           0x00020000);
-}
-template <bool kRows>
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t v_rsrc(const QueryTile &t) {
-  const int keys = kRows ? t.kend : (((t.kend - 1) >> 5) + 1) * kBlock;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(t.vc), 0, uint32_t(keys) * (D * 2),
-                                           0x00020000);
+// past its last block) give zeros; the scores of those keys are masked. Their
+// 32-bit range and offsets end at kMaxRange keys, so the key-split tile, which
+// any cache may take, has a buffer per 32-key block.
+constexpr int kMaxRange = (1 << 24) - kBlock;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t key_rsrc(const u32x4 *base, int first, int keys) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(base) + size_t(first) * (D / 8), 0,
+                                           uint32_t(keys) * (D * 2), 0x00020000);
 }
 
 // V of a 32-key block staged as it lies in memory, 8 KiB either way.
@@ -175,20 +172,20 @@ __device__ __forceinline__ void attn_query_tile(const QueryTile &t, float qscale
   const int r = lane >> 4, i = lane & 15;
   const int nblk = t.blk1 ? t.blk1 : (t.kend + kBlock - 1) / kBlock;  // blocks [blk0, nblk)
   const int first = t.blk0 + wave;
-  const auto rk = k_rsrc(t), rv = v_rsrc<kRows>(t);
   u32x4 *ks = sh.kv[wave][0], *vs = sh.kv[wave][1];
   auto fetch = [&](int kb) {
-    const uint32_t base = uint32_t(kb) * (D * 2);
+    const int keys = min(kBlock, t.kend - kb);
+    const auto rk = key_rsrc(t.kc, kb, keys), rv = key_rsrc(t.vc, kb, kRows ? keys : kBlock);
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rk, (lds_ptr_t)(ks + 64 * q), 16,
-          base + uint32_t((4 * q + r) * (D * 2) + (i ^ (4 * (q >> 1) + r)) * 16), 0, 0, 0);
+          uint32_t((4 * q + r) * (D * 2) + (i ^ (4 * (q >> 1) + r)) * 16), 0, 0, 0);
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rv, (lds_ptr_t)(vs + 64 * q), 16,
-          base + (kRows ? v_row_fetch(lane, q) : v_block_fetch(lane, q)), 0, 0, 0);
+          kRows ? v_row_fetch(lane, q) : v_block_fetch(lane, q), 0, 0, 0);
   };
   if (first < nblk)
     fetch(first * kBlock);
@@ -359,7 +356,8 @@ __device__ __forceinline__ void attn_query_tile64(const QueryTile &t, float qsca
       qb[s] = src[4 * s + r];
   }
   const int kmax = t.causal_pos >= 0 ? t.causal_pos + 16 * wave + i : t.kv_len - 1;
-  const auto rk = k_rsrc(t), rv = v_rsrc<kRows>(t);
+  const auto rk = key_rsrc(t.kc, 0, t.kend);
+  const auto rv = key_rsrc(t.vc, 0, kRows ? t.kend : (t.kend + kBlock - 1) / kBlock * kBlock);
   // this wave's quarter of the N blocks at kb0 into `stage`: K pieces 2 w,
   // 2 w + 1 (T = w / 2, s = 2 (w % 2) + {0, 1}) and V dim tiles 2 w, 2 w + 1.
   // Keys are clamped to the last visible one.
@@ -548,7 +546,10 @@ inline TilePlan attn_tile_plan(long long heads, int q_len, int kv_len, bool caus
       best_t = t;
     }
   };
+  const bool far = kv_len > kMaxRange;  // past the 64-query tile's buffers
   for (const Form &f : causal ? tri : whole) {
+    if (far && f.queries == 64)
+      continue;
     const int blocks = f.queries == 64 ? f.blocks : f.waves, per_cu = f.slots / 256;
     const long long tiles = heads * ((q_len + f.queries - 1) / f.queries);
     const long long steps = (nb + blocks - 1) / blocks, total = tiles * steps;
@@ -557,7 +558,7 @@ inline TilePlan attn_tile_plan(long long heads, int q_len, int kv_len, bool caus
       return f.alone +
              (per_cu == 1 ? 0.0 : (f.full - f.alone) * double((n - 1) / 256) / (per_cu - 1));
     };
-    if (f.queries == 64 || tiles <= (heads <= 64 ? 1536 : 512)) {
+    if (f.queries == 64 || far || tiles <= (heads <= 64 ? 1536 : 512)) {
       const long long full = tiles / f.slots, rem = tiles % f.slots;
       const double rate = double(full) * f.full + (rem ? step(rem) : 0.0);
       if (causal) {
