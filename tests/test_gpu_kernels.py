@@ -486,7 +486,7 @@ def test_gemm_split_k_matches_oracle(torch, yuear_lib, oracle, m, n, k, residual
 
 
 # tokens, features, K and epilogue that take each shape of the one-round form
-# on 256 CUs (gemm_ksplit_choice): ragged tiles in both directions, K of one
+# on 256 CUs (gemm_pick): ragged tiles in both directions, K of one
 # step (one wave has work), of fewer steps than waves, and of uneven shares
 @pytest.mark.parametrize("m,n,k,residual", [
     (1, 100, 64, 0), (1, 99, 1600, 1), (49, 1028, 1600, 2), (66, 1027, 64, 1), (97, 2052, 576, 2),
@@ -494,6 +494,8 @@ def test_gemm_split_k_matches_oracle(torch, yuear_lib, oracle, m, n, k, residual
     (301, 3075, 576, 0), (131, 6150, 576, 2), (257, 4100, 192, 1), (301, 4099, 192, 0),
     (513, 3076, 192, 1), (400, 4100, 576, 2), (700, 3075, 192, 0), (1010, 3070, 64, 2),
     (700, 4100, 576, 1),
+    # ... the largest shapes, which win at longer K only
+    (700, 3075, 1600, 0), (1010, 3070, 2048, 2), (295, 8200, 3072, 1),
 ])
 def test_gemm_few_tokens(torch, yuear_lib, oracle, m, n, k, residual):
     """The K-split form of the GEMM (gemm_ksplit.hip) against the oracle on

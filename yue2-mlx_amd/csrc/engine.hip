@@ -968,21 +968,13 @@ void prefill(yuear_session &S, int b, const int32_t *ids, int n, uint16_t *logit
     // h: a split GEMM's reduce and the norm run as one kernel (bit-identical to
     // the reduce kernel followed by the norm)
     auto residual_then_norm = [&](GemmParams g, const uint16_t *norm_w) -> hipError_t {
-      const int few = gemm_ksplit_choice(g.m, g.n, g.k, gemm_cus());
-      if (few >= 0) {
-        const hipError_t e = launch_gemm_ksplit(g, few, st);
-        return e != hipSuccess
-                   ? e
-                   : launch_rms_norm_rows(S.px, T, c.H, norm_w, c.eps, S.ph, st);
-      }
-      int shape = 0, splits = 1;
-      gemm_plan(g.m, g.n, g.k, gemm_cus(), g.part_bytes, &shape, &splits);
-      const bool fuse = splits > 1 && S.fuse_norm;
+      const GemmPick pick = gemm_pick(g.m, g.n, g.k, gemm_cus(), g.part_bytes);
+      const bool fuse = pick.splits > 1 && S.fuse_norm;
       g.defer_reduce = fuse;
-      hipError_t e = launch_gemm_tile(g, shape, st, splits);
+      const hipError_t e = launch_gemm_pick(g, pick, st);
       if (e != hipSuccess)
         return e;
-      return fuse ? launch_gemm_reduce_norm(g, splits, norm_w, c.eps, S.ph, st)
+      return fuse ? launch_gemm_reduce_norm(g, pick.splits, norm_w, c.eps, S.ph, st)
                   : launch_rms_norm_rows(S.px, T, c.H, norm_w, c.eps, S.ph, st);
     };
     HIPC(launch_rms_norm_rows(S.px, T, c.H, E.layers[0].input_ln, c.eps, S.ph, st));

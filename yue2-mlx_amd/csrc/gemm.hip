@@ -29,9 +29,9 @@
 // the 256 x 256 tile were conflict stalls). Fragment of a 16-wide K sub-step
 // s: lane l reads row l % 32, chunk 2 s + l / 32.
 //
-// Tile shapes (past the sizes that gemm_ksplit.hip does in one round of
-// smaller tiles, launch_gemm picks the one with the least estimated time for
-// the shape and the CU count): 256 x 256 (8 waves of 128 x 64), 256 x 128 and
+// Tile shapes (launch_gemm picks the one with the least estimated time for the
+// problem and the CU count, or a form of gemm_ksplit.hip where one round of smaller
+// tiles is estimated faster): 256 x 256 (8 waves of 128 x 64), 256 x 128 and
 // 128 x 256 (8 waves of 64 x 64), 256 x 192 (8 waves of 64 x 96), 192 x 192
 // (8 waves of 96 x 48) and 128 x 128 (4 waves of 64 x 64, two workgroups per
 // CU); all but the last on 16 x 16 x 32 MFMAs (gemm_tile16 below), that one
@@ -460,29 +460,23 @@ YUEAR_GEMM_KERNEL(gemm_128x128, gemm_tile, 128, 128, 2, 2)
 YUEAR_GEMM_KERNEL(gemm_192x192, gemm_tile16, 192, 192, 2, 4)
 #undef YUEAR_GEMM_KERNEL
 
-// Time model of the tile shapes, in microseconds per 48 K steps on MI355X (K =
-// 3072, 256 CUs): `alone` for a tile with a CU to itself on an otherwise idle
-// chip, `busy` with every CU holding one such tile, `round` for a full round of
-// per_cu workgroups on every CU. kShapes: fitted to all six shapes on eight
-// projections (2048-16384 rows, K 2048-8192) at 17 token counts from 140 to 3000,
-// weights from HBM; its pick takes 0.14% more than the fastest shape on average
-// (4% at worst; kWarmShapes, fitted with the weights in cache, 1.9% and 18%: 301
-// x 16384 x 3072 65 us against 57, 2500 x 16384 x 3072 253 against 224).
-// kWarmShapes weighs splits of K (gemm_plan), with whose costs it was fitted.
+// Time model of the tile shapes, in us on MI355X (256 CUs), as {fixed, per 1024 of
+// K}: `alone` for a tile with a CU to itself on an otherwise idle chip, `busy` with
+// every CU holding one such tile, `round` for a full round of per_cu workgroups on
+// every CU. Fitted with the weights in HBM; see gemm_pick.
 struct TileShape {
   int bm, bn, per_cu;
-  double alone, busy, round;
+  double alone[2], busy[2], round[2];
 };
 constexpr TileShape kShapes[] = {
-    {256, 256, 1, 65.7, 86.7, 83.5}, {256, 128, 1, 47.2, 58.8, 53.7},
-    {128, 256, 1, 41.3, 68.9, 60.9}, {256, 192, 1, 57.7, 72.0, 70.1},
-    {128, 128, 2, 38.5, 46.5, 53.6}, {192, 192, 1, 49.6, 61.3, 59.9},
+    {256, 256, 1, {34.78, 23.05}, {3.61, 21.24}, {7.559, 18.31}},
+    {256, 128, 1, {5.87, 23.67}, {6.668, 15.47}, {6.166, 15.37}},
+    {128, 256, 1, {1.863, 124}, {4.599, 14.02}, {4.8, 20.72}},
+    {256, 192, 1, {12.07, 20.38}, {9.082, 20.03}, {6.011, 18.76}},
+    {128, 128, 2, {7.364, 9.731}, {5.586, 10.15}, {16.99, 13.88}},
+    {192, 192, 1, {16.76, 20.02}, {6.907, 15.15}, {6.782, 19.09}},
 };
-constexpr TileShape kWarmShapes[] = {
-    {256, 256, 1, 63.0, 85.0, 85.0}, {256, 128, 1, 43.5, 50.0, 50.0},
-    {128, 256, 1, 44.3, 50.0, 50.0}, {256, 192, 1, 49.0, 58.0, 58.0},
-    {128, 128, 2, 34.3, 40.0, 50.8}, {192, 192, 1, 41.0, 49.0, 49.0},
-};
+constexpr int kNumShapes = int(sizeof(kShapes) / sizeof(kShapes[0]));
 
 // Split-K: the sum over the splits in split order (a fixed order: the result
 // does not depend on which split finished first), then the epilogue; one
@@ -656,77 +650,58 @@ hipError_t launch_tile(void (*kern)(GemmParams, int, int), const GemmParams &p, 
   return hipGetLastError();
 }
 
-int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus < 1)
-    cus = 256;
-  return cus;
-}
-
 }  // namespace
 
-int gemm_tile_choice(int m, int n, int cus) {
-  int best = 0;
-  double best_t = 0;
-  for (int i = 0; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
-    const TileShape &t = kShapes[i];
-    const long long tiles = (long long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-    const long long slots = (long long)cus * t.per_cu;
-    const long long full = tiles / slots, rem = tiles % slots;
-    // full rounds, then a last round that is cheaper the fewer CUs it loads
-    double time = double(full) * t.round;
-    if (rem > cus)
-      time += t.round;
-    else if (rem > 0)
-      time += t.alone + (t.busy - t.alone) * double(rem) / cus;
-    if (i == 0 || time < best_t * 0.999) {
-      best = i;
-      best_t = time;
-    }
-  }
-  return best;
+namespace {
+// us of m x n x k by tiles of shape t with K in z ranges, without the reduce:
+// full rounds, then a last round that is cheaper the fewer CUs it loads
+double tile_time(const TileShape &t, int m, int n, int k, int z, int cus) {
+  const long long wgs = (long long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn) * z;
+  const long long slots = (long long)cus * t.per_cu, full = wgs / slots, rem = wgs % slots;
+  const double kk = double(k) / z / 1024;
+  auto us = [&](const double (&c)[2]) { return c[0] + c[1] * kk; };
+  double time = double(full) * us(t.round);
+  if (rem > cus)
+    time += us(t.round);
+  else if (rem > 0)
+    time += us(t.alone) + (us(t.busy) - us(t.alone)) * double(rem) / cus;
+  return time;
 }
+}  // namespace
 
-// Shape and split count together, by the tile model scaled to K / splits
-// steps, plus, for a split, the reduce kernel: 4 us and 0.4 us per MB it
-// moves (the splits' fp32 partials read, the bf16 result written) and 0.1 us
-// per MB of partials the tiles write instead of bf16 results. Fitted to
-// every (shape, splits) of the four 3B prefill projections at 128-2048
-// tokens on MI355X: the pick is within 9% of the fastest measured (split or
-// not) in all 28 cases; without a split it is gemm_tile_choice's shape.
-void gemm_plan(int m, int n, int k, int cus, size_t part_bytes, int *shape, int *splits) {
-  const int whole = gemm_tile_choice(m, n, cus);
-  *shape = whole;
-  *splits = 1;
-  double best_t = 0;
+// The form of least time by the models of the whole-K tiles (above), of the
+// K-split tiles (gemm_ksplit_choice) and, with a workspace, of whole-K tiles with
+// K split over workgroups: the tiles at K / splits, then 5.6 us, 0.46 us per MB the
+// reduce kernel moves (the splits' fp32 partials read, the bf16 result written) and
+// 0.018 us per MB of partials the tiles write. Fitted on MI355X with weights from
+// HBM to 3800 shapes (9-4096 tokens, 64-16384 features, K 64-8192, all epilogues),
+// the six tiles each, 350 of them with all splits: without a workspace the pick is
+// 0.2% from the fastest on average (14% at worst), with one 0.6% (14%). Models
+// fitted at K 3072 only picked launches 1.6 times as slow as the best at K 64-512
+// (200 x 16384 x 256: 13.2 us against 9.0) and 1.2-1.3 times at K 1024 (2000 x
+// 2048 x 1024: 19 against 16).
+GemmPick gemm_pick(int m, int n, int k, int cus, size_t part_bytes) {
+  GemmPick pick;
+  double best = __builtin_inf();
+  const int few = gemm_ksplit_choice(m, n, k, cus, &best);
+  if (few >= 0)
+    pick = GemmPick{true, few, 1};
   const double mn = double(m) * double(n);
-  for (int i = 0; i < int(sizeof(kShapes) / sizeof(kShapes[0])); ++i) {
-    const TileShape &t = kWarmShapes[i];
-    const long long tiles = (long long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-    const long long slots = (long long)cus * t.per_cu;
+  for (int i = 0; i < kNumShapes; ++i)
     for (int z = 1; z <= kMaxSplits; ++z) {
       // whole 64-wide steps, at least 4 per split, the partials in the workspace
-      if ((k / kBK) % z || k / z < 4 * kBK ||
-          (z > 1 && size_t(m) * size_t(n) > part_bytes / (size_t(z) * 4)))
+      if (z > 1 && ((k / kBK) % z || k / z < 4 * kBK ||
+                    size_t(m) * size_t(n) > part_bytes / (size_t(z) * 4)))
         continue;
-      const long long wgs = tiles * z, full = wgs / slots, rem = wgs % slots;
-      double round = double(full) * t.round;
-      if (rem > cus)
-        round += t.round;
-      else if (rem > 0)
-        round += t.alone + (t.busy - t.alone) * double(rem) / cus;
-      double time = round * (double(k) / z / kBK) / 48.0;
+      double time = tile_time(kShapes[i], m, n, k, z, cus);
       if (z > 1)
-        time += 4.0 + 0.4e-6 * (4.0 * z * mn + 2.0 * mn) + 0.1e-6 * 4.0 * z * mn;
-      if ((i == 0 && z == 1) || time < best_t * 0.999) {
-        *shape = z > 1 ? i : whole;
-        *splits = z;
-        best_t = time;
+        time += 5.6 + 0.46e-6 * (4.0 * z * mn + 2.0 * mn) + 0.018e-6 * 4.0 * z * mn;
+      if (time < best * 0.999) {
+        pick = GemmPick{false, i, z};
+        best = time;
       }
     }
-  }
+  return pick;
 }
 
 hipError_t launch_gemm_tile(const GemmParams &p, int shape, hipStream_t s, int splits) {
@@ -759,19 +734,24 @@ hipError_t launch_gemm_reduce_norm(const GemmParams &p, int splits, const uint16
   return hipGetLastError();
 }
 
-int gemm_cus() { return device_cus(); }
+int gemm_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 1)
+    cus = 256;
+  return cus;
+}
 
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s) {
-  const int cus = device_cus();
-  if (p.m > 0 && p.n > 0 && p.k >= kBK) {
-    const int few = gemm_ksplit_choice(p.m, p.n, p.k, cus);
-    if (few >= 0)
-      return launch_gemm_ksplit(p, few, s);
-  }
-  int shape = gemm_tile_choice(p.m, p.n, cus), splits = 1;
-  if (p.part)
-    gemm_plan(p.m, p.n, p.k, cus, p.part_bytes, &shape, &splits);
-  return launch_gemm_tile(p, shape, s, splits);
+  if (p.m < 1 || p.n < 1 || p.k < kBK)
+    return hipErrorInvalidValue;
+  return launch_gemm_pick(p, gemm_pick(p.m, p.n, p.k, gemm_cus(), p.part ? p.part_bytes : 0), s);
+}
+
+hipError_t launch_gemm_pick(const GemmParams &p, const GemmPick &pick, hipStream_t s) {
+  return pick.few ? launch_gemm_ksplit(p, pick.shape, s)
+                  : launch_gemm_tile(p, pick.shape, s, pick.splits);
 }
 
 }  // namespace yuear

@@ -218,9 +218,11 @@ constexpr int kNumShapes = int(sizeof(kShapes) / sizeof(kShapes[0]));
 // projections of both decoder widths on MI355X with cold weights: the pick is
 // within 0.8% of the fastest on average, within 14% always. Past one round the
 // 128-wide tiles read fewer bytes per product: gate/up at 301 tokens 61 us in
-// two rounds, 56 with 256 x 128 tiles; within one round this form is the
-// faster one at every measured size but 2048 x 2048 x 2048 (26.7 / 25.1 us).
-int gemm_ksplit_choice(int m, int n, int k, int cus) {
+// two rounds, 56 with 256 x 128 tiles. Within one round they win at short K, whose
+// sums over the waves cost more than the products (700 x 4096 x 256: 9.4 us, 8.6
+// with 128 x 128 tiles): *us is the estimate that gemm_pick compares, fitted with
+// theirs.
+int gemm_ksplit_choice(int m, int n, int k, int cus, double *us) {
   int best = -1;
   double best_t = 0;
   for (int i = 0; i < kNumShapes; ++i) {
@@ -230,11 +232,13 @@ int gemm_ksplit_choice(int m, int n, int k, int cus) {
     const int per_cu = s.lds() <= 80 * 1024 ? 2 : 1;
     if (tiles > (long long)cus * per_cu)
       continue;
-    const double each = double(bm + bn) * k * 2e-3 / 86.0 + 0.17 * s.mt * s.nb;
-    const double t = tiles > cus ? 2 * each : each;
+    const double kb = double(bm + bn) * k * 2e-3;  // KB of rows a tile reads
+    const int rounds = tiles > cus ? 2 : 1;
+    const double t = rounds * (kb / 86.0 + 0.17 * s.mt * s.nb);
     if (best < 0 || t < best_t) {
       best = i;
       best_t = t;
+      *us = 1.215 + rounds * (kb / 74.7 + 0.1482 * s.mt * s.nb + 0.7085);
     }
   }
   return best;

@@ -181,19 +181,25 @@ struct GemmParams {
   bool defer_reduce = false;
 };
 // MFMA GEMM (gemm.hip); k a multiple of 64, lda a multiple of 8. With a
-// workspace it may split K over workgroups (gemm_plan picks the tile shape
-// and split count together), summing the splits in a fixed order.
+// workspace it may split K over workgroups, summing the splits in a fixed order.
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s);
+// The form launch_gemm takes for m x n x k on `cus` CUs with a workspace of
+// part_bytes: shape `shape` of the K-split form (few; gemm_ksplit.hip) or of the
+// whole-K tiles with K in `splits` ranges.
+struct GemmPick {
+  bool few = false;
+  int shape = 0, splits = 1;
+};
+GemmPick gemm_pick(int m, int n, int k, int cus, size_t part_bytes);
+hipError_t launch_gemm_pick(const GemmParams &p, const GemmPick &pick, hipStream_t s);
 // One of the GEMM's tile shapes (0..5, see gemm.hip) with K in `splits`
 // ranges (splits > 1 needs p.part of splits * m * n floats, k / 64 a multiple
-// of splits), the shape launch_gemm would pick for m x n on `cus` CUs, and
-// its split count.
+// of splits).
 hipError_t launch_gemm_tile(const GemmParams &p, int shape, hipStream_t s, int splits = 1);
-int gemm_tile_choice(int m, int n, int cus);
 // The K-split form (gemm_ksplit.hip) for GEMMs that fit one round of its
-// tiles: the shape to launch, or -1 when there is none. launch_gemm takes it
-// first. No workspace; the sums' order depends on k and the shape only.
-int gemm_ksplit_choice(int m, int n, int k, int cus);
+// tiles: the shape to launch and its estimated time, or -1 when there is none. No
+// workspace; the sums' order depends on k and the shape only.
+int gemm_ksplit_choice(int m, int n, int k, int cus, double *us);
 hipError_t launch_gemm_ksplit(const GemmParams &p, int shape, hipStream_t s);
 int gemm_cus();  // CUs of the current device (256 if it cannot be read)
 // The reduce of a residual GEMM launched with defer_reduce and splits > 1
@@ -203,7 +209,6 @@ int gemm_cus();  // CUs of the current device (256 if it cannot be read)
 // residual 1, n a multiple of 8 up to 8192, ldc == n.
 hipError_t launch_gemm_reduce_norm(const GemmParams &p, int splits, const uint16_t *norm_w,
                                    float eps, uint16_t *y, hipStream_t s);
-void gemm_plan(int m, int n, int k, int cus, size_t part_bytes, int *shape, int *splits);
 
 // dst[0..n) = w.v[0..n), n <= 8; elems bf16 (a multiple of 8) of `src` to
 // pinned host memory.
