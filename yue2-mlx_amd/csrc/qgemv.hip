@@ -219,6 +219,8 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
   // 4. Row set blk, or with LOOP blk, blk + gridDim.x, ...: the next set's
   // loads are issued before this one's products, and no barrier separates the
   // sets (a wave's sums pass through its own part of `res`).
+  static_assert(B * R * RW <= 64, "one lane per (row, branch) of a wave");
+  static_assert(R * RW % 2 == 0 || R * RW == 1, "a wave's rows are whole pairs, or one");
   float *own = &res[0][0] + wave * (R * RW * B);  // [B][R * RW]
   auto products = [&](int buf, int set) {
     float acc[R][B];
@@ -305,6 +307,15 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
         const int b = lane / (R * RW / 2), i = lane % (R * RW / 2), row = row0 + 2 * i;
         if (b < B && row + 1 < p.n) {
           const float g = rbf(own[b * (R * RW) + 2 * i]), u = rbf(own[b * (R * RW) + 2 * i + 1]);
+          const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
+          p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
+        }
+      } else if constexpr (!LOOP) {  // one row a wave: a pair's rows are in two waves
+        __syncthreads();
+        const float *gate = &res[0][0] + (tid & 1) * (2 * B), *up = gate + B;  // [wave][B]
+        const int b = tid >> 1, row = set * ROWS + 2 * (tid & 1);
+        if (b < B && row + 1 < p.n) {
+          const float g = rbf(gate[b]), u = rbf(up[b]);
           const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
           p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
         }
@@ -397,6 +408,7 @@ hipError_t launch_lp(const GemvParams &p, hipStream_t s) {
         if (sets(2) >= 512)
           return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
       }
+      // (SwiGLU needs a pair's rows in one wave, or the barrier of the one-pass form)
       if (sets(1) > 512 && (L < 64 || p.epilogue != kEpiSwiGLU))
         return launch_r<B, BITS, L, P, 1, true>(p, s, 512);
     }
@@ -407,10 +419,6 @@ hipError_t launch_lp(const GemvParams &p, hipStream_t s) {
   }
   if constexpr (P <= 4) {
     if (sets(2) >= 1024)
-      return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
-  }
-  if constexpr (L == 64) {  // a (gate, up) pair stays in one wave
-    if (p.epilogue == kEpiSwiGLU)
       return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
   }
   return launch_r<B, BITS, L, P, 1, false>(p, s, sets(1));
