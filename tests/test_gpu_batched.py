@@ -132,3 +132,38 @@ def test_sample_rejects_batched_sessions(engine):
     with pytest.raises(ValueError, match="independently"):
         s.sample(GREEDY, 1, 0)
     s.close()
+
+
+@pytest.mark.parametrize("hidden", [6144, 8192])
+def test_batched_wide_hidden_prepares_rows_once(yuear_lib, hidden):
+    """Sessions of 3+ sequences of a model wider than 3072: the normed projections
+    take the row kernel's buffer (every workgroup normalising 6144 or 8192 wide
+    rows for itself is the slower form), and each sequence gets the logits of a
+    session of its own."""
+    import torch
+    cfg = dict(hidden_size=hidden, intermediate_size=512, num_hidden_layers=1, num_attention_heads=4,
+               num_key_value_heads=2, head_dim=128, vocab_size=512, max_position_embeddings=64,
+               rms_norm_eps=1e-5, rope_theta=500000.0, qk_norm=True)
+    engine = yuear_lib.Engine(cfg, yuear_lib.random_weights(cfg, 4, 0.02, 0.1))
+    ids = np.random.default_rng(hidden).integers(0, 512, (3, 9))
+    s = engine.session(3, 16)
+    for b in range(3):
+        s.prefill(b, ids[b, :8].tolist())
+    got = s.step(ids[:, 8].tolist())
+    import cpu_ref
+    for b in range(3):
+        one = engine.session(1, 16)
+        one.prefill(0, ids[b, :8].tolist())
+        want = cpu_ref.bf16_to_f32(one.step(int(ids[b, 8]))[0])
+        err = np.abs(cpu_ref.bf16_to_f32(got[b]) - want)
+        assert (err <= 2e-2 + 1e-2 * np.abs(want)).all(), (b, err.max())
+        one.close()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        for which in ("qkv", "gate_up", "lm_head"):
+            s.time_kernel(which, 1)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert any("gemv_mfma_kernel" in n for n in names), names
+    assert sum(e.count for e in prof.key_averages() if "stage_rows_kernel" in e.key) == 6, names
+    s.close()
+    engine.close()

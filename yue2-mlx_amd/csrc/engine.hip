@@ -275,6 +275,7 @@ struct yuear_session {
   uint16_t *kc = nullptr, *vc = nullptr;
   int32_t *pos = nullptr, *tok = nullptr;
   uint16_t *x = nullptr, *qkv = nullptr, *attn = nullptr, *act = nullptr, *logits = nullptr;
+  uint16_t *stage = nullptr;  // [B][H] rows of the batched GEMVs that need it (gemv_mfma_staged)
   float *part_o = nullptr, *part_ml = nullptr;
   int32_t *counters = nullptr;
   float *scratch = nullptr, *alphas = nullptr;
@@ -629,6 +630,8 @@ void begin_session(yuear_session &S, yuear_engine *E, int branches, int capacity
   HIPC(hipMemsetAsync(S.pos, 0, branches * 4, S.stream));
   HIPC(hipMemsetAsync(S.tok, 0, branches * 4, S.stream));
   S.x = S.alloc<uint16_t>(size_t(branches) * c.H);
+  if (branches >= 3 && c.H > 3072)
+    S.stage = S.alloc<uint16_t>(size_t(branches) * c.H);
   S.qkv = S.alloc<uint16_t>(size_t(branches) * c.qkv());
   S.attn = S.alloc<uint16_t>(size_t(branches) * c.Hq * c.D);
   S.act = S.alloc<uint16_t>(size_t(branches) * c.F);
@@ -736,6 +739,7 @@ void enqueue_layer(yuear_session &S, int l, bool embed_first) {
   }
   q.norm_w = L.input_ln;
   q.eps = c.eps;
+  q.stage = S.stage;
   q.w_tiled = L.qkv_t;
   q.y = S.qkv;
   q.y_stride = c.qkv();
@@ -805,6 +809,7 @@ void enqueue_ffn(yuear_session &S, int l, uint16_t *x, int batch) {
   g.x_stride = c.H;
   g.norm_w = L.post_ln;
   g.eps = c.eps;
+  g.stage = S.stage;
   g.w_tiled = L.gu_t;
   g.y = S.act;
   g.y_stride = c.F;
@@ -842,6 +847,7 @@ void enqueue_head(yuear_session &S, const uint16_t *x, int batch, int x_stride, 
   h.x_stride = x_stride;
   h.norm_w = E.final_norm;
   h.eps = c.eps;
+  h.stage = S.stage;
   h.w_tiled = E.lm_head_t;
   h.y = out;
   h.y_stride = S.phase.stride();
@@ -861,6 +867,7 @@ void enqueue_one(yuear_session &S, const std::string &which, int l) {
   GemvParams g;
   g.batch = S.B;
   g.eps = c.eps;
+  g.stage = S.stage;
   if (which == "qkv") {
     g.w = L.qkv; g.n = c.qkv(); g.k = c.H; g.x = S.x; g.x_stride = c.H;
     set_quant(g, E.bits, L.qqkv, L.gqkv);
@@ -1701,10 +1708,8 @@ int32_t yuear_op_gemv(const uint16_t *w, int32_t n, int32_t k, int32_t batch, co
   p.epilogue = epilogue;
   const uint16_t *x_end = x + size_t(std::max(batch, 1) - 1) * std::max(x_stride, 0) + std::max(k, 0);
   const uint16_t *y_end = y + size_t(std::max(batch, 1) - 1) * std::max(y_stride, 0) + std::max(n, 0);
-  if (batch >= 3 && norm_w && k > 0 && (k > 3072 || (x < y_end && y < x_end))) {
-    // the batched form normalises the rows into a buffer first: in place; or
-    // of a k whose workgroups would repeat it too often (3072 x 8192, 8 rows,
-    // 16 us; by every workgroup 25)
+  if (gemv_mfma_staged(p) || (batch >= 3 && norm_w && k > 0 && x < y_end && y < x_end)) {
+    // the batched form normalises the rows into a buffer first
     static OpPool pool;
     void *stage = nullptr;
     bool fresh = false;

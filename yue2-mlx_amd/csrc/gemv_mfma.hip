@@ -44,9 +44,9 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast
 
 // Rows prepared in a buffer of their own (grid = batch rows, 256 threads), where
 // the caller gives one: y may then overlap x (workgroups read x while others
-// write y), and with k of 6144 or more it is faster (3072 x 8192, 8 rows, 16
-// against 25 us: a workgroup's only tiles wait for the norm). Gather from the embedding (copy-out to x_out) and/or RMSNorm with the
-// rounding points of ar.cpp:30-35, written to p.stage.
+// write y), and normed rows of more than 3072 are faster so (gemv_mfma_staged).
+// Gather from the embedding (copy-out to x_out) and/or RMSNorm with the rounding
+// points of ar.cpp:30-35, written to p.stage.
 __global__ __launch_bounds__(256) void stage_rows_kernel(GemvParams p) {
   __shared__ float red[4];
   constexpr int kMaxChunks = 4;  // k <= 8192
@@ -395,8 +395,14 @@ bool gemv_mfma_supported(const GemvParams &p) {
          (p.epilogue != kEpiSwiGLU || p.n % 2 == 0);
 }
 
+// Every workgroup would repeat the norm of 6144 or 8192 wide rows while its only
+// tiles wait (3072 x 8192, 8 rows: 25 us, 16 with the row kernel before it).
+bool gemv_mfma_staged(const GemvParams &p) {
+  return gemv_mfma_supported(p) && p.norm_w && p.k > 3072;
+}
+
 hipError_t launch_gemv_mfma(const GemvParams &p, hipStream_t s) {
-  if (!gemv_mfma_supported(p) || p.n < 1)
+  if (!gemv_mfma_supported(p) || p.n < 1 || (gemv_mfma_staged(p) && !p.stage))
     return hipErrorInvalidValue;
   if (!p.stage || (!p.norm_w && !p.embed && !p.x_out))
     return launch_k(p, s);

@@ -33,8 +33,9 @@ struct GemvParams {
   int epilogue = kEpiStore;
   int seg0_start = 0, seg0_len = 1 << 30, seg1_start = 0;  // row map
   int32_t *advance = nullptr;  // block 0 increments advance[0..batch)
-  // optional [batch][k] scratch of the batched (MFMA) form: with it a row kernel
-  // first writes the gathered / normalised rows there (y may then overlap x).
+  // [batch][k] scratch of the batched (MFMA) form: with it a row kernel first
+  // writes the gathered / normalised rows there (y may then overlap x). Required
+  // where gemv_mfma_staged() says so.
   uint16_t *stage = nullptr;
   // The same weight rows in the MFMA-tiled layout of launch_tile_rows, read
   // by the batched form when given.
@@ -64,6 +65,8 @@ void quantize_affine(const uint16_t *w, int64_t rows, int k, int bits, uint32_t 
 // MFMA form for 3..8 independent rows (batched sequences); launch_gemv
 // dispatches to it when gemv_mfma_supported(p).
 bool gemv_mfma_supported(const GemvParams &p);
+// The launch needs p.stage: the row kernel is the faster prologue.
+bool gemv_mfma_staged(const GemvParams &p);
 hipError_t launch_gemv_mfma(const GemvParams &p, hipStream_t s);
 // Copy W [n][k] (k a multiple of 32) into the MFMA-tiled layout: for each
 // 16-row tile t and 32-column step s, 1 KiB whose 16-byte piece l is row
