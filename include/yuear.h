@@ -243,8 +243,9 @@ yuear_status yuear_session_time_kernel(yuear_session *session,
  * one needing a larger buffer) allocates, so make it outside graph capture;
  * yuear_op_gemm and yuear_op_gemm_tile use no scratch. The first SwiGLU
  * GEMM (residual 2) on a device fills a 128 KiB silu table (one launch and a
- * stream synchronisation): make it outside graph capture too, where it
- * returns hipErrorStreamCaptureUnsupported. ---- */
+ * stream synchronisation): make it outside graph capture too, where calls
+ * whose tiles read the table return hipErrorStreamCaptureUnsupported (the
+ * smallest ones do not need it and run). ---- */
 /* y[b][r] = bf16(x[b] . W[row(r)]) with optional RMSNorm prologue
  * (norm_w != NULL) and epilogue 0 store / 1 residual add / 2 SwiGLU pairs. */
 int32_t yuear_op_gemv(const uint16_t *dev_w, int32_t n, int32_t k,

@@ -724,3 +724,55 @@ def test_attention_prefill_past_2_24_keys(torch, yuear_lib):
         ref = e @ f(kv[1][see]) / (e.sum() + pos0 + t + 1 - len(see))
         # the sum of 2^24 equal weights in fp32 partial sums of 2^17 each
         np.testing.assert_allclose(got[t], ref, rtol=2 ** -7, atol=2 ** -8 * np.abs(ref).max())
+
+
+SILU_CHILD = """
+import ctypes, sys, torch
+sys.path.insert(0, sys.argv[1])
+import yuear
+k, n = 192, 8192
+a = torch.randn(3000, k, device="cuda").bfloat16()
+w = torch.randn(n, k, device="cuda").bfloat16()
+c, d = (torch.zeros(3000, n // 2, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+s = torch.cuda.Stream()
+def gemm(m, out):
+    return yuear.lib.yuear_op_gemm(a.data_ptr(), k, w.data_ptr(), m, n, k, out.data_ptr(), n // 2, 2,
+                                   s.cuda_stream)
+with torch.cuda.stream(s):
+    g = torch.cuda.CUDAGraph()
+    if sys.argv[2] == "small first":
+        assert gemm(32, c) == 0
+    else:  # the smallest forms need no table and may be a device's first call
+        with torch.cuda.graph(g, stream=s):
+            assert gemm(32, c) == 0
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        status = gemm(3000, c)
+    print("captured", status, flush=True)
+    if sys.argv[2] == "small first":
+        assert status == 0
+        assert gemm(3000, d) == 0
+        for _ in range(2):
+            c.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, d)
+    else:
+        assert status != 0
+print("ok")
+"""
+
+
+@pytest.mark.parametrize("order", ["small first", "captured first"])
+def test_small_swiglu_gemm_prepares_a_capture(yuear_lib, order):
+    """A device's first SwiGLU GEMM fills the silu table also where it takes the
+    form without one, so that a large one can be captured next; inside a capture
+    the small form runs without the table. A process of its own: the table is
+    filled once per device and process."""
+    import os
+    import subprocess
+    import sys
+    run = subprocess.run([sys.executable, "-c", SILU_CHILD, os.path.dirname(yuear_lib.__file__), order],
+                         capture_output=True, text=True, timeout=90)
+    assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout + run.stderr[-2000:]

@@ -750,6 +750,13 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s) {
 }
 
 hipError_t launch_gemm_pick(const GemmParams &p, const GemmPick &pick, hipStream_t s) {
+  if (pick.few && p.residual == 2) {
+    // The K-split form reads no silu table, but a first SwiGLU call made to
+    // prepare for a capture is to fill it whatever its size.
+    const hipError_t e = ensure_silu_table(s);
+    if (e != hipSuccess && e != hipErrorStreamCaptureUnsupported)
+      return e;
+  }
   return pick.few ? launch_gemm_ksplit(p, pick.shape, s)
                   : launch_gemm_tile(p, pick.shape, s, pick.splits);
 }
