@@ -61,3 +61,22 @@ def test_mfma_operand_tuples_intact(source, tmp_path):
         problems += [(name, b) for b in bad]
     assert total > 0, "no MFMA found"
     assert not problems, problems[:3]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) and not shutil.which("hipcc"), reason="no hipcc")
+def test_batched_gemv_kernels_do_not_spill(tmp_path):
+    """The batched projections' kernels (up to 1024 threads, so 128 registers a lane)
+    keep weights and activations in registers: nothing of theirs goes to scratch."""
+    out = tmp_path / "gemv_mfma.s"
+    run = subprocess.run([HIPCC, *FLAGS, os.path.join(CSRC, "gemv_mfma.hip"), "-o", str(out)],
+                         capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0, run.stderr[-2000:]
+    kernels, name = {}, None
+    for line in out.read_text().splitlines():
+        key, _, value = line.strip().partition(":")
+        if key == ".name" and value.strip().startswith("_Z"):
+            name = value.strip()
+        elif key == ".vgpr_spill_count":
+            kernels[name] = int(value)
+    assert sum("gemv_mfma_kernel" in k for k in kernels) >= 10
+    assert not {k: v for k, v in kernels.items() if v}

@@ -133,12 +133,16 @@ struct Shape {
   }
 };
 
+// The widest rows that a workgroup gathers and normalises itself.
+constexpr int kMaxOwnRows = 3072;
+
 // LOOP: a workgroup walks the sets of T tiles blockIdx + i gridDim.
 template <int KW, int STEPS, int T, bool LOOP, int EPI>
 __global__ __launch_bounds__(KW * T * 64) void gemv_mfma_kernel(GemvParams p) {
   extern __shared__ u32x4 lds[];
   using S = Shape<KW, STEPS, T>;
   constexpr int K = S::K, NCH = S::NCH, G = S::G, R = (8 + G - 1) / G;
+  constexpr bool kPlain = K > kMaxOwnRows;  // x is prepared: no gather, no norm
   const int B = p.batch;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -152,12 +156,13 @@ __global__ __launch_bounds__(KW * T * 64) void gemv_mfma_kernel(GemvParams p) {
   for (int i = 0; i < R; ++i) {
     const int b = grp + G * i;
     if (grp < G && b < B) {
-      const uint16_t *src = p.embed ? p.embed + size_t(min(max(p.tokens[b], 0), p.embed_rows - 1)) * K
-                                    : p.x + size_t(b) * p.x_stride;
+      const uint16_t *src = !kPlain && p.embed
+                                ? p.embed + size_t(min(max(p.tokens[b], 0), p.embed_rows - 1)) * K
+                                : p.x + size_t(b) * p.x_stride;
       xr[i] = reinterpret_cast<const u32x4 *>(src)[c];
     }
   }
-  if (p.norm_w && grp < G)
+  if (!kPlain && p.norm_w && grp < G)
     gain = reinterpret_cast<const u32x4 *>(p.norm_w)[c];
   // keep these loads ahead of the weight stream (the scheduler may otherwise
   // sink some below it, and the staging would then wait for every weight)
@@ -187,13 +192,13 @@ __global__ __launch_bounds__(KW * T * 64) void gemv_mfma_kernel(GemvParams p) {
   }
 
   // 3. gather copy-out, RMSNorm, staging
-  if (p.x_out && blockIdx.x == 0) {
+  if (!kPlain && p.x_out && blockIdx.x == 0) {
 #pragma unroll
     for (int i = 0; i < R; ++i)
       if (grp < G && grp + G * i < B)
         reinterpret_cast<u32x4 *>(p.x_out + size_t(grp + G * i) * p.x_stride)[c] = xr[i];
   }
-  if (p.norm_w) {
+  if (!kPlain && p.norm_w) {
 #pragma unroll
     for (int i = 0; i < R; ++i)
       if (grp < G && grp + G * i < B) {
@@ -336,7 +341,9 @@ hipError_t launch_shape(const GemvParams &p, hipStream_t s) {
 // a CU twice, one round of those (12288 x 2048: 11.2 us, the loop 12.4). Normed
 // rows take the threads of another tile even so (4096 x 2048, 8 rows: 8.7 us with
 // one tile, 6.7 with two; 1024 x 3072 10.1 with two, 9.2 with three). K of 6144
-// and more is a single workgroup per CU: 16 waves on one tile, or on two.
+// and more is a single workgroup per CU: 16 waves on one tile, or on two (its rows
+// are always prepared, so its 128 registers a lane hold the weights of 16 steps:
+// 101, where the gather and norm code made it spill 12-29 of them).
 hipError_t launch_k(const GemvParams &p, hipStream_t s) {
   const int tiles = (p.n + 7) / 8;
   const bool norm = p.norm_w != nullptr;
@@ -398,7 +405,7 @@ bool gemv_mfma_supported(const GemvParams &p) {
 // Every workgroup would repeat the norm of 6144 or 8192 wide rows while its only
 // tiles wait (3072 x 8192, 8 rows: 25 us, 16 with the row kernel before it).
 bool gemv_mfma_staged(const GemvParams &p) {
-  return gemv_mfma_supported(p) && p.norm_w && p.k > 3072;
+  return gemv_mfma_supported(p) && (p.norm_w || p.embed || p.x_out) && p.k > kMaxOwnRows;
 }
 
 hipError_t launch_gemv_mfma(const GemvParams &p, hipStream_t s) {
