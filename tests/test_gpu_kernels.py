@@ -114,6 +114,21 @@ def test_gemv_batched_tiles(torch, yuear_lib, oracle, n, k, batch, norm, epilogu
     test_gemv_matches_oracle(torch, yuear_lib, oracle, n, k, batch, norm, epilogue)
 
 
+@pytest.mark.parametrize("k", [2048, 3072, 6144, 8192])
+@pytest.mark.parametrize("n", [8, 9, 16])
+def test_gemv_batched_few_outputs_in_place(torch, yuear_lib, k, n):
+    # without a norm: up to 16 outputs are one workgroup's, which may lie over x
+    rng = np.random.default_rng(k + n)
+    w, x = bf(rng.normal(size=(n, k)) / k ** 0.5), bf(rng.normal(size=(8, k)))
+    dw, dx, dy = (dev(torch, a) for a in (w, x, np.zeros_like(x)))
+    for y in (dy, dx):
+        assert yuear_lib.lib.yuear_op_gemv(dw.data_ptr(), n, k, 8, dx.data_ptr(), k, None, 1e-5,
+                                           y.data_ptr(), k, 0, None) == 0
+    got = host(torch, dx)
+    np.testing.assert_array_equal(got[:, :n], host(torch, dy)[:, :n])
+    np.testing.assert_array_equal(got[:, n:], x[:, n:])
+
+
 @pytest.mark.parametrize("k", [2048, 3072])
 def test_gemv_batched_in_place(torch, yuear_lib, oracle, k):
     # y over x: the workgroups must not read rows that others have written
@@ -776,3 +791,16 @@ def test_small_swiglu_gemm_prepares_a_capture(yuear_lib, order):
     run = subprocess.run([sys.executable, "-c", SILU_CHILD, os.path.dirname(yuear_lib.__file__), order],
                          capture_output=True, text=True, timeout=90)
     assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stdout + run.stderr[-2000:]
+
+
+@pytest.mark.parametrize("m,k", [(1, 64), (40, 128), (300, 128), (1000, 192), (700, 256)])
+def test_gemm_in_place(torch, yuear_lib, m, k):
+    """C over A, up to one tile of features wide: no workgroup may read rows that
+    another has written. Against the same product into a buffer of its own."""
+    rng = np.random.default_rng(m)
+    a, w = bf(rng.normal(size=(m, k))), bf(rng.normal(size=(k, k)) / k ** 0.5)
+    dw, da, dc = dev(torch, w), dev(torch, a), dev(torch, np.zeros((m, k), np.uint16))
+    for c in (dc, da):
+        assert yuear_lib.lib.yuear_op_gemm(da.data_ptr(), k, dw.data_ptr(), m, k, k, c.data_ptr(), k, 0,
+                                           None) == 0
+    assert_close_bf16(host(torch, da), host(torch, dc), exact_frac=0.9)

@@ -746,6 +746,23 @@ int gemm_cus() {
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s) {
   if (p.m < 1 || p.n < 1 || p.k < kBK)
     return hipErrorInvalidValue;
+  // c over a (rows of one stride, at most one tile of features wide): a workgroup
+  // reads all of its rows before it writes them, so one column of whole-K tiles
+  // may work in place
+  const size_t out_n = p.residual == 2 ? p.n / 2 : p.n;
+  if (p.n <= 256 && p.a < p.c + size_t(p.m - 1) * p.ldc + out_n &&
+      p.c < p.a + size_t(p.m - 1) * p.lda + p.k) {
+    GemmPick pick;
+    double best = __builtin_inf();
+    for (int i = 0; i < kNumShapes; ++i) {
+      const double t = tile_time(kShapes[i], p.m, p.n, p.k, 1, gemm_cus());
+      if (kShapes[i].bn >= p.n && t < best) {
+        pick.shape = i;
+        best = t;
+      }
+    }
+    return launch_gemm_pick(p, pick, s);
+  }
   return launch_gemm_pick(p, gemm_pick(p.m, p.n, p.k, gemm_cus(), p.part ? p.part_bytes : 0), s);
 }
 

@@ -346,24 +346,26 @@ hipError_t launch_shape(const GemvParams &p, hipStream_t s) {
 // 101, where the gather and norm code made it spill 12-29 of them).
 hipError_t launch_k(const GemvParams &p, hipStream_t s) {
   const int tiles = (p.n + 7) / 8;
-  const bool norm = p.norm_w != nullptr;
+  // rows of one tile a workgroup; two tiles are one workgroup, which has read all of
+  // x before it writes: up to 16 outputs may lie over x
+  const bool norm = p.norm_w != nullptr, single = tiles <= 256 && tiles != 2;
   switch (p.k) {
   case 2048:
-    return tiles <= 256 && !norm ? launch_shape<4, 8, 1>(p, s)
-           : tiles <= 512        ? launch_shape<4, 8, 2>(p, s)
-           : tiles <= 768        ? launch_shape<4, 8, 3>(p, s)
-           : tiles <= 1024       ? launch_shape<4, 8, 4>(p, s)
-           : tiles <= 1536       ? launch_shape<4, 8, 3>(p, s)
-                                 : launch_shape<4, 8, 2, true>(p, s);
+    return single && !norm ? launch_shape<4, 8, 1>(p, s)
+           : tiles <= 512  ? launch_shape<4, 8, 2>(p, s)
+           : tiles <= 768  ? launch_shape<4, 8, 3>(p, s)
+           : tiles <= 1024 ? launch_shape<4, 8, 4>(p, s)
+           : tiles <= 1536 ? launch_shape<4, 8, 3>(p, s)
+                           : launch_shape<4, 8, 2, true>(p, s);
   case 3072:
     return tiles <= 512 && !norm ? launch_shape<4, 12, 2>(p, s)
            : tiles <= 768        ? launch_shape<4, 12, 3>(p, s)
            : tiles <= 1024       ? launch_shape<4, 12, 4>(p, s)
                                  : launch_shape<4, 12, 2, true>(p, s);
   case 6144:
-    return tiles <= 256 ? launch_shape<16, 6, 1>(p, s) : launch_shape<8, 12, 2>(p, s);
+    return single ? launch_shape<16, 6, 1>(p, s) : launch_shape<8, 12, 2>(p, s);
   case 8192:
-    return tiles <= 256 ? launch_shape<16, 8, 1>(p, s) : launch_shape<8, 16, 2>(p, s);
+    return single ? launch_shape<16, 8, 1>(p, s) : launch_shape<8, 16, 2>(p, s);
   }
   return hipErrorInvalidValue;
 }
