@@ -210,3 +210,32 @@ def test_nar_attention_graph_survives_a_larger_call(torch, yuear_lib):
             np.testing.assert_array_equal(host(torch, out), want, err_msg=f"replay {replay}")
     again = host(torch, yuear_lib.nar_attention(*large, workspace=ws, stream=s.cuda_stream))
     np.testing.assert_array_equal(again, big)
+
+
+def test_nar_attention_threads_share_a_stream(torch, yuear_lib):
+    """Dealt calls of two threads on one stream share its pool buffer: a call's
+    attention and merge are enqueued as one, so that neither reads the other's
+    partial sums."""
+    import threading
+    rng = np.random.default_rng(5)
+    sets = [[dev(torch, bf(rng.normal(size=(1, h, n, 128)))) for h, n in ((16, 100), (8, 8001), (8, 8001))]
+            for _ in range(2)]
+    want = [yuear_lib.nar_attention(*s) for s in sets]
+    torch.cuda.synchronize()
+    got, errors = [[], []], []
+
+    def work(i):
+        try:
+            got[i] += [yuear_lib.nar_attention(*sets[i]) for _ in range(60)]
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for i in range(2):
+        for out in got[i]:
+            assert torch.equal(out, want[i])

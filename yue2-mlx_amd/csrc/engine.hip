@@ -1140,17 +1140,18 @@ void check_sampler_phase(yuear_session &S, double cfg_scale) {
 namespace {
 // Scratch of the op-level entry points, one buffer per (device, stream):
 // calls on one stream are ordered and may share it, calls on different
-// streams or devices never do. Grown on demand (the stream is synchronised
-// before the smaller buffer is freed), kept until the process ends.
-// Scratch of the op-level entry points, one buffer per (device, stream). A
-// buffer handed out is never freed: a launch still in flight, or a graph
-// captured on that stream, may hold its address. A request larger than the
+// streams or devices never do. A buffer handed out is never freed: a launch
+// still in flight, or a graph captured on that stream, may hold its address. A
+// request larger than the
 // current buffer retires it (kept until the process ends) and allocates
 // max(request, 2 x current) rounded to a power of two, so a growing caller
 // retires O(log size) buffers and never synchronises. Growth while the
 // stream is being captured is refused (hipErrorStreamCaptureUnsupported):
 // make the largest call once before capturing.
 struct OpPool {
+  // Held by a call from get() to its last launch where several launches pass data
+  // through the buffer: two threads' calls on one stream must not interleave them.
+  std::mutex enqueue;
   std::mutex mu;
   std::map<std::pair<int, hipStream_t>, std::pair<void *, size_t>> bufs;
   std::vector<void *> retired;
@@ -1711,6 +1712,7 @@ int32_t yuear_op_gemv(const uint16_t *w, int32_t n, int32_t k, int32_t batch, co
   if (gemv_mfma_staged(p) || (batch >= 3 && norm_w && k > 0 && x < y_end && y < x_end)) {
     // the batched form normalises the rows into a buffer first
     static OpPool pool;
+    std::lock_guard<std::mutex> hold(pool.enqueue);
     void *stage = nullptr;
     bool fresh = false;
     const hipError_t e = pool.get(static_cast<hipStream_t>(stream), size_t(batch) * k * 2, &stage,
@@ -1825,11 +1827,13 @@ yuear_status yuear_nar_attention(const uint16_t *q, const uint16_t *k, const uin
     p.q = q;
     p.k = k;
     p.v = v;
+    static OpPool pool;
+    std::unique_lock<std::mutex> hold(pool.enqueue, std::defer_lock);
     // partials of dealt launches, from a per-(device, stream) pool. Without
     // them (a capture cannot allocate; no memory) whole tiles run.
     const size_t pf = nar_attention_part_floats(batch, heads, q_len, kv_len, causal != 0);
     if (pf) {
-      static OpPool pool;
+      hold.lock();
       void *buf = nullptr;
       bool fresh = false;
       const hipError_t e = pool.get(static_cast<hipStream_t>(stream), pf * 4, &buf, &fresh);
@@ -1918,13 +1922,15 @@ int32_t yuear_op_gemm_split(const uint16_t *a, int32_t lda, const uint16_t *w, i
                             int32_t shape, int32_t splits, void *stream) {
   GemmParams p{a, lda, w, m, n, k, c, ldc, residual};
   const hipStream_t st = static_cast<hipStream_t>(stream);
+  static OpPool pool;
+  std::unique_lock<std::mutex> hold(pool.enqueue, std::defer_lock);
   if (splits > 1) {
     // the checks launch_gemm_tile repeats, before anything is allocated
     // (m * n below 2^58 keeps the workspace size within size_t)
     if (m < 1 || n < 1 || splits > 16 || k < 64 || k % 64 || (k / 64) % splits ||
         size_t(m) * size_t(n) > (SIZE_MAX >> 6))
       return int32_t(hipErrorInvalidValue);
-    static OpPool pool;
+    hold.lock();
     void *buf = nullptr;
     bool fresh = false;
     const size_t bytes = size_t(splits) * size_t(m) * size_t(n) * 4;
