@@ -346,8 +346,8 @@ int32_t yuear_op_attention_prefill(const uint16_t *dev_q,
  * otherwise, nar_attention.cpp:245-268). This entry point computes those
  * with the same precise kernel too: their parity with the reference is
  * unpinned. workspace: yuear_nar_attention_workspace_bytes()
- * of device memory (required; the kernels of this version read V as given and
- * leave it untouched). Non-causal launches may deal the keys of a query tile
+ * of device memory (required; V is read as given, and copied there only where
+ * out lies over it). Non-causal launches may deal the keys of a query tile
  * to several workgroups; their partials (at most 35 MB) come from a library
  * pool per (device, stream). So the first such call on a stream, or one that
  * needs a larger pool, allocates: make it outside graph capture, where such a

@@ -239,3 +239,25 @@ def test_nar_attention_threads_share_a_stream(torch, yuear_lib):
     for i in range(2):
         for out in got[i]:
             assert torch.equal(out, want[i])
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "q shifted"])
+@pytest.mark.parametrize("heads,n,lk", [(2, 64, 2100), (48, 300, 300)])
+def test_nar_attention_output_over_an_input(torch, yuear_lib, which, heads, n, lk):
+    """Output written over the queries, keys or values: workgroups that still read
+    them must not see it. Dealt and whole tiles, against separate buffers."""
+    import ctypes as C
+    rng = np.random.default_rng(n)
+    q, k, v = (dev(torch, bf(rng.normal(size=(1, heads, m, 128)))) for m in (n, lk, lk))
+    want = host(torch, yuear_lib.nar_attention(q, k, v))
+    room = torch.zeros(heads * n * 128 + 4096, dtype=torch.bfloat16, device="cuda")
+    room[4096:] = q.view(-1)
+    out = {"q": room[4096:], "q shifted": room, "k": k, "v": v}[which]
+    ws = torch.empty(yuear_lib.lib.yuear_nar_attention_workspace_bytes(1, heads, lk) // 2,
+                     dtype=torch.bfloat16, device="cuda")
+    err = C.c_void_p()
+    assert yuear_lib.lib.yuear_nar_attention(room.data_ptr() + 8192, k.data_ptr(), v.data_ptr(), 1, heads,
+                                             heads, n, lk, 128, 0, 64, ws.data_ptr(), out.data_ptr(), None,
+                                             C.byref(err)) == 0
+    got = host(torch, out.view(-1)[:heads * n * 128]).reshape(want.shape)
+    np.testing.assert_array_equal(got, want)

@@ -1852,7 +1852,37 @@ yuear_status yuear_nar_attention(const uint16_t *q, const uint16_t *k, const uin
     p.q_len = q_len;
     p.kv_len = kv_len;
     p.causal = causal != 0;
-    HIPC(launch_nar_attention(p, static_cast<hipStream_t>(stream)));
+    // Workgroups write out while others still read K and V (queries are read by
+    // those that write their rows): inputs that out lies over are copied first, V
+    // into the workspace.
+    const size_t q_elems = size_t(batch) * heads * q_len * 128;
+    const size_t kv_elems = size_t(batch) * kv_heads * kv_len * 128;
+    auto over = [&](const uint16_t *t, size_t n) { return t < out + q_elems && out < t + n; };
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    static OpPool copies;
+    const bool copy_q = q != out && over(q, q_elems), copy_k = over(k, kv_elems);
+    std::unique_lock<std::mutex> hold_copies(copies.enqueue, std::defer_lock);
+    if (copy_q || copy_k) {
+      hold_copies.lock();
+      void *buf = nullptr;
+      bool fresh = false;
+      HIPC(copies.get(st, ((copy_q ? q_elems : 0) + (copy_k ? kv_elems : 0)) * 2, &buf, &fresh));
+      uint16_t *to = static_cast<uint16_t *>(buf);
+      if (copy_q) {
+        HIPC(launch_copy_out(to, q, q_elems, st));
+        p.q = to;
+        to += q_elems;
+      }
+      if (copy_k) {
+        HIPC(launch_copy_out(to, k, kv_elems, st));
+        p.k = to;
+      }
+    }
+    if (over(v, kv_elems)) {
+      HIPC(launch_copy_out(static_cast<uint16_t *>(workspace), v, kv_elems, st));
+      p.v = static_cast<uint16_t *>(workspace);
+    }
+    HIPC(launch_nar_attention(p, st));
   });
 }
 

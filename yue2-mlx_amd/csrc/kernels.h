@@ -214,7 +214,7 @@ hipError_t launch_gemm_reduce_norm(const GemmParams &p, int splits, const uint16
                                    float eps, uint16_t *y, hipStream_t s);
 
 // dst[0..n) = w.v[0..n), n <= 8; elems bf16 (a multiple of 8) of `src` to
-// pinned host memory.
+// pinned host or device memory.
 struct Words {
   int32_t v[8];
 };
