@@ -3,12 +3,14 @@
 Invariant: every register of an MFMA's A or B operand tuple carries the value
 the kernel's source gave that tuple. Walking back from the MFMA, each
 register's value comes either from a load that wrote the whole tuple (a
-global, buffer or LDS load; read-modify-writes of the register in between,
+global, buffer or LDS load, or two transposing LDS reads of one operand, its
+halves 1024 bytes apart from one address; read-modify-writes of the register in between,
 such as the decode attention's current-key insert or its value mask, keep
 that origin) or from VALU instructions that built the tuple register by
 register (the P pieces). A tuple whose registers mix both origins, or come
 from different loads, has had part of a loaded operand overwritten before
-the MFMA read it.
+the MFMA read it. A register that an MFMA wrote last is a raw score (or sum),
+never a bf16 operand.
 
 This catches a register-allocation error of the ROCm 7.2 compiler seen in
 the decode attention's earlier source: with the P split through
@@ -55,19 +57,31 @@ def _writes(op, ops):
 
 
 def _origin(insts, idx, reg):
-    j = idx - 1
+    j, built = idx - 1, False
     while j >= 0:
         op, ops = insts[j]
         if op.startswith("v_mfma") and reg in _regs(ops[0]):
-            return ("valu", j)  # a score, from which the P pieces are made
+            # a score: the P pieces are made from it, in place or not
+            return ("valu" if built else "mfma", j)
         if reg in _writes(op, ops):
             if op.startswith(_LOADS):
                 return ("load", j)
             if reg not in _regs(",".join(ops[1:])):
                 return ("valu", j)
-            # a read-modify-write keeps the register's origin
+            built = True  # a read-modify-write keeps the register's origin
         j -= 1
     return ("entry", -1)
+
+
+def _tr_pair(lo, hi):
+    """Two transposing LDS reads of one operand: keys 0-3 and, 1024 bytes on from
+    the same address, keys 4-7 of a dim tile. (The address register may have been
+    moved from one to the other; its name is what the listing shows.)"""
+    def at(inst):
+        m = re.search(r"offset:(\d+)", inst[1][1])
+        return inst[1][1].split()[0], int(m.group(1)) if m else 0
+    (la, lo_ofs), (ha, hi_ofs) = at(lo), at(hi)
+    return la == ha and hi_ofs - lo_ofs == 1024
 
 
 def functions(asm_text):
@@ -102,9 +116,10 @@ def check_function(lines):
             # two transposing LDS reads build a tuple, one half each
             if (kinds == {"load"} and len(loads) == 2 and len(regs) == 4 and
                     all(insts[j][0].startswith("ds_read_b64_tr") for j in loads) and
-                    origins[0] == origins[1] and origins[2] == origins[3]):
+                    origins[0] == origins[1] and origins[2] == origins[3] and
+                    _tr_pair(insts[origins[0][1]], insts[origins[2][1]])):
                 continue
-            if ("load" in kinds and len(kinds) > 1) or len(loads) > 1:
+            if ("load" in kinds and len(kinds) > 1) or len(loads) > 1 or "mfma" in kinds:
                 bad.append((op + " " + ", ".join(ops),
                             [(k, " ".join([insts[j][0]] + insts[j][1]) if j >= 0 else "")
                              for k, j in origins]))

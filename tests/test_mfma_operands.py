@@ -47,6 +47,44 @@ def test_checker_flags_an_overwritten_operand_register():
     assert len(bad) == 1 and "v[6:9]" in bad[0][0]
 
 
+TRANSPOSED = """_Zk:
+	ds_read_b64_tr_b16 v[2:3], v10 offset:8192
+	ds_read_b64_tr_b16 v[4:5], v10 offset:9216
+	ds_read_b64_tr_b16 v[6:7], v10 offset:8224
+	ds_read_b64_tr_b16 v[8:9], v10 offset:9248
+	v_mfma_f32_16x16x32_bf16 v[20:23], v[40:43], v[44:47], 0
+	v_perm_b32 v30, v21, v20, s0
+	v_and_b32_e32 v20, 0xffff0000, v20
+	v_perm_b32 v20, v21, v20, s0
+	v_mov_b32_e32 v31, v30
+	v_mov_b32_e32 v32, v30
+	v_mov_b32_e32 v33, v30
+	v_mfma_f32_16x16x32_bf16 a[0:3], v[2:5], v[30:33], a[0:3]
+	v_mfma_f32_16x16x32_bf16 a[4:7], v[6:9], v[30:33], a[4:7]
+.Lfunc_end0:
+"""
+
+
+def test_checker_on_transposed_reads_and_scores():
+    def check(text):
+        return mfma_operands.check_function(text.splitlines()[1:])
+    count, bad = check(TRANSPOSED)
+    assert count == 3 and not bad
+    # halves of two dim tiles in one operand, in either order
+    for a, b in (("v[4:5], v10 offset:9216", "v[4:5], v10 offset:9248"),
+                 ("v[2:3], v10 offset:8192", "v[2:3], v10 offset:8224"),
+                 ("v[4:5], v10 offset:9216", "v[4:5], v11 offset:9216")):
+        assert a in TRANSPOSED
+        _, bad = check(TRANSPOSED.replace(a, b))
+        assert len(bad) == 1 and "v[2:5]" in bad[0][0], (a, bad)
+    # a register of P still holds the raw score
+    _, bad = check(TRANSPOSED.replace("a[4:7], v[6:9], v[30:33]", "a[4:7], v[6:9], v[21:24]"))
+    assert len(bad) == 1 and "v[21:24]" in bad[0][0]
+    # ... or was split in place: a built piece
+    built = TRANSPOSED.replace("v_mov_b32_e32 v31, v30", "v_mov_b32_e32 v31, v20")
+    assert not check(built)[1]
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC) and not shutil.which("hipcc"), reason="no hipcc")
 @pytest.mark.parametrize("source", SOURCES)
 def test_mfma_operand_tuples_intact(source, tmp_path):
