@@ -68,17 +68,18 @@ def test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, 
     # than waves, a partial last block, a last tile of one query
     (1, 1, 1, 1, 31, False), (2, 6, 3, 17, 289, False), (1, 1, 1, 1, 697, False),
     (1, 6, 3, 677, 919, False), (1, 24, 8, 300, 1100, False), (1, 24, 8, 250, 3600, False),
-    (1, 24, 8, 1001, 1500, False),
+    (1, 24, 8, 1001, 1500, False), (1, 24, 8, 341, 1500, False),
     # dealt to all CUs: key-split tiles of 16 and 32 queries by 8 waves, steps
     # and blocks that do not divide, a ragged last tile
     (2, 16, 8, 1, 4001, False), (1, 16, 8, 53, 2000, False), (1, 24, 8, 53, 6500, False),
     (1, 6, 3, 274, 6000, False), (1, 16, 8, 100, 8001, False),
-    # ... to fewer workgroups, as few keys or heads allow: 8, 56, 72, 104, 208
+    # ... to fewer workgroups, as few keys or heads allow: 8, 56, 64, 104, 208, 24
     (1, 1, 1, 1, 20000, False), (1, 1, 1, 100, 2000, False), (1, 2, 1, 33, 8001, False),
     (1, 2, 2, 130, 1500, False), (1, 16, 8, 17, 12001, False), (1, 1, 1, 65, 1500, False),
-    # ... 4 waves, 264 and 360 workgroups; 64-query tiles, an odd last block
-    (1, 1, 1, 341, 3001, False), (1, 6, 2, 65, 3001, False), (1, 24, 8, 341, 1500, False),
-    (1, 2, 1, 341, 6001, False),
+    # ... 4 waves, 264 and 360 workgroups of 16 queries, 256 of 32; 64-query tiles, an
+    # odd last block
+    (1, 1, 1, 341, 3001, False), (1, 6, 2, 65, 3001, False), (1, 2, 1, 341, 6001, False),
+    (1, 24, 8, 500, 3470, False),
     # 64-query tiles, one and two blocks a step, an odd last block; causal forms
     (1, 12, 4, 677, 31, False), (1, 24, 8, 1024, 400, False), (1, 48, 16, 1025, 97, False),
     (1, 24, 8, 1001, 289, False), (1, 24, 8, 100, 100, True),
@@ -102,9 +103,38 @@ def test_nar_attention_large_scores(torch, yuear_lib, mag, Hq, Hkv, Lq, Lk, caus
     np.testing.assert_array_equal(host(torch, got)[0], want)
 
 
-def test_nar_attention_zero_pads_the_last_key_block(torch, yuear_lib, oracle):
-    # 50 keys leave 14 padding slots in the last 32-key block of the
-    # workspace: a workspace full of NaN must not reach the output
+# (heads, kv heads, queries, keys), each with a last key block that is not full:
+# key-split tiles of 16 and 32 queries by 4 and 8 waves, dealt, 64-query tiles by one
+# and two blocks a step (an odd number of blocks)
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lk", [
+    (2, 2, 9, 70), (2, 2, 1, 697), (16, 2, 257, 289), (6, 3, 677, 919), (2, 2, 100, 2001),
+    (16, 8, 100, 8001), (24, 2, 341, 1505), (24, 8, 500, 3470), (96, 2, 257, 31),
+    (24, 2, 1001, 289),
+])
+def test_nar_attention_reads_no_neighbouring_keys(torch, yuear_lib, oracle, Hq, Hkv, Lq, Lk):
+    """The last key block of a kv head lies over the next head's first rows, and of the
+    last head past the tensor: NaN and inf there (weights 0 times them would be NaN) must
+    not reach the head's queries."""
+    rng = np.random.default_rng(Lk)
+    per = Hq // Hkv
+    q = bf(rng.normal(size=(1, Hq, Lq, 128)))
+    for good in (0, Hkv - 1):  # the one head with numbers in it
+        k, v = (np.full(((Hkv + 1) * Lk * 128 + 4096,), 0x7FC0, np.uint16) for _ in range(2))
+        v[::3] = 0x7F80
+        kv = [bf(rng.normal(size=(1, 1, Lk, 128))) for _ in range(2)]
+        at = 2048 + good * Lk * 128  # (rows before the first head are NaN too)
+        k[at:at + Lk * 128], v[at:at + Lk * 128] = (t.reshape(-1) for t in kv)
+        dk, dv = dev(torch, k), dev(torch, v)
+        got = host(torch, yuear_lib.nar_attention(
+            dev(torch, q), dk[2048:2048 + Hkv * Lk * 128].view(1, Hkv, Lk, 128),
+            dv[2048:2048 + Hkv * Lk * 128].view(1, Hkv, Lk, 128)))
+        mine = slice(good * per, good * per + per)
+        ref = oracle.nar_attention(q[:, mine], *kv)
+        assert_close_bf16(got[:, mine], ref, exact_frac=0.8)
+
+
+def test_nar_attention_leaves_the_workspace(torch, yuear_lib, oracle):
+    # V is read as given: the workspace is neither read (NaN) nor written
     rng = np.random.default_rng(1)
     q = bf(rng.normal(size=(1, 4, 20, 128)))
     k = bf(rng.normal(size=(1, 2, 50, 128)))
@@ -114,9 +144,8 @@ def test_nar_attention_zero_pads_the_last_key_block(torch, yuear_lib, oracle):
     ws = dev(torch, np.full(nbytes // 2, 0x7FC0, np.uint16))
     got = host(torch, yuear_lib.nar_attention(dev(torch, q), dev(torch, k), dev(torch, v),
                                               workspace=ws))
-    import cpu_ref
-    assert not np.isnan(cpu_ref.bf16_to_f32(got)).any()
     assert_close_bf16(got, oracle.nar_attention(q, k, v), exact_frac=0.8)
+    assert (host(torch, ws) == 0x7FC0).all()
 
 
 def test_nar_attention_errors(torch, yuear_lib):
@@ -181,22 +210,33 @@ def test_nar_condition_is_the_prefill_cache(torch, yuear_lib, oracle):
     q.close()
 
 
+def merges(torch, call):
+    """Merge kernels that `call` launches: a dealt launch has one."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return sum(e.count for e in prof.key_averages() if "nar_merge_kernel" in e.key)
+
+
+def nar_inputs(torch, rng, hq, hkv, lq, lk):
+    return [bf(rng.normal(size=(1, h, n, 128))) for h, n in ((hq, lq), (hkv, lk), (hkv, lk))]
+
+
 def test_nar_attention_graph_survives_a_larger_call(torch, yuear_lib):
-    """The split partials come from a pool per (device, stream). A graph
-    captured on a stream keeps the pool buffer it was captured with: a later
+    """The partials of a dealt launch come from a pool per (device, stream). A
+    graph captured on a stream keeps the pool buffer it was captured with: a later
     call on that stream that needs a larger buffer allocates a new one and
     keeps the old one alive, so replays of the graph stay correct."""
     rng = np.random.default_rng(21)
-
-    def inputs(lk):
-        return (dev(torch, bf(rng.normal(size=(1, 16, 64, 128)))),
-                dev(torch, bf(rng.normal(size=(1, 8, lk, 128)))),
-                dev(torch, bf(rng.normal(size=(1, 8, lk, 128)))))
-
-    small, large = inputs(600), inputs(2570)  # 2 and 9 key splits
+    # 256 workgroups x 2 pieces of 16 and of 32 queries: 4.3 and 8.7 MB, over and
+    # under the 8 MB that the pool's first buffer rounds up to
+    small = [dev(torch, a) for a in nar_inputs(torch, rng, 16, 8, 64, 2570)]
+    large = [dev(torch, a) for a in nar_inputs(torch, rng, 6, 3, 274, 6000)]
+    for args in (small, large):
+        assert merges(torch, lambda: yuear_lib.nar_attention(*args)) == 1
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
-        ws = torch.empty(yuear_lib.lib.yuear_nar_attention_workspace_bytes(1, 8, 2570) // 2,
+        ws = torch.empty(yuear_lib.lib.yuear_nar_attention_workspace_bytes(1, 8, 6000) // 2,
                          dtype=torch.bfloat16, device="cuda")
         want = yuear_lib.nar_attention(*small, workspace=ws, stream=s.cuda_stream)
         want = host(torch, want)
@@ -210,6 +250,29 @@ def test_nar_attention_graph_survives_a_larger_call(torch, yuear_lib):
             np.testing.assert_array_equal(host(torch, out), want, err_msg=f"replay {replay}")
     again = host(torch, yuear_lib.nar_attention(*large, workspace=ws, stream=s.cuda_stream))
     np.testing.assert_array_equal(again, big)
+
+
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lk", [(16, 8, 64, 2570), (1, 1, 1, 20000), (24, 8, 500, 3470)])
+def test_nar_attention_captured_before_its_pool(torch, yuear_lib, oracle, Hq, Hkv, Lq, Lk):
+    """A dealt shape captured on a stream that has no pool buffer yet: the capture
+    cannot allocate, so whole tiles run."""
+    args = nar_inputs(torch, np.random.default_rng(Lk), Hq, Hkv, Lq, Lk)
+    ref = oracle.nar_attention(*args)
+    args = [dev(torch, a) for a in args]
+    assert merges(torch, lambda: yuear_lib.nar_attention(*args)) == 1
+    s = torch.cuda.Stream()
+    ws = torch.empty(yuear_lib.lib.yuear_nar_attention_workspace_bytes(1, Hkv, Lk) // 2,
+                     dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        out = yuear_lib.nar_attention(*args, workspace=ws, stream=s.cuda_stream)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert_close_bf16(host(torch, out), ref, exact_frac=0.8)
+    assert merges(torch, g.replay) == 0
 
 
 def test_nar_attention_threads_share_a_stream(torch, yuear_lib):
