@@ -41,16 +41,16 @@ def host(torch, t):
     (1, 4, 4, 40, 1, False),       # one key
     (1, 16, 8, 257, 257, True),    # causal conditioning prefill
     (2, 6, 3, 64, 64, True),
-    # >= 768 workgroups of 64 queries: the LDS-shared 64-query tile (ragged last tiles)
+    # whole 64-query tiles, one or two key blocks a step (ragged last tiles)
     (2, 24, 8, 1000, 1100, False),
     (1, 24, 8, 2050, 2050, True),
     (32, 24, 8, 64, 1, False),     # 768 workgroups of 64 queries over one key
     (16, 24, 8, 130, 130, True),   # 1152 workgroups, causal, 2-query last tiles
-    # keys split over workgroups (fewer than 768 workgroups of 64 queries)
-    (1, 16, 8, 64, 2570, False),   # 81 key blocks: 9 splits of 9, none empty
+    # keys dealt over workgroups
+    (1, 16, 8, 64, 2570, False),   # 16-query tiles, 81 key blocks
     (1, 24, 8, 512, 3512, False),  # the benchmarked acoustic chunk over conditioning keys
-    (1, 16, 8, 4, 3100, False),    # 4 queries in one 64-query tile, 12 splits
-    (2, 16, 8, 100, 1500, False),  # batch 2, 5 splits, ragged last query tile
+    (1, 16, 8, 4, 3100, False),    # 4 queries in one tile, 12-13 workgroups a tile
+    (2, 16, 8, 100, 1500, False),  # batch 2, whole key-split tiles, ragged last one
 ])
 def test_nar_attention_matches_oracle(torch, yuear_lib, oracle, B, Hq, Hkv, Lq, Lk, causal):
     print(f"[nar] B={B} Hq={Hq} Hkv={Hkv} Lq={Lq} Lk={Lk} causal={causal}", flush=True)

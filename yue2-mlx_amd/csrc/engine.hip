@@ -92,9 +92,9 @@ const char *const kLayerNames[] = {"input_layernorm",  "post_attention_layernorm
                                    "mlp.down_proj"};
 constexpr int kNumLayerTensors = 11;
 // Split-K workspace of a session's prefill GEMMs (fp32 partials, splits x
-// tokens x features): the largest split the plan picks at the 3B shape is
-// the down projection at 1024 tokens, 4 x 1024 x 3072 floats (48 MiB); a
-// split that does not fit is not considered.
+// tokens x features): the largest split that gemm_pick takes at the 3B shape is
+// the down projection's at 2048 tokens, 2 x 2048 x 3072 floats (48 MiB); a split
+// that does not fit is not considered.
 constexpr size_t kSplitBytes = size_t(64) << 20;
 
 int32_t tensor_id(const std::string &name) {
@@ -241,8 +241,9 @@ struct yuear_engine {
   uint32_t *qweights = nullptr;  // codes and group words of every quantized linear
   const uint32_t *lm_q = nullptr, *lm_g = nullptr;
   // MFMA-tiled projection copies, built by the first session of 3+ branches
-  // (6.15 GB more at the 3B shape: HBM is plentiful, the batched GEMVs read
-  // 1 KiB contiguous per wave-load from them)
+  // (6.15 GB more at the 3B shape: steps of 3 and 8 sequences are 1-2% faster
+  // from them than from the rows, 3072 wide 1.501 and 1.744 ms against 1.531 and
+  // 1.760; of 5 even)
   uint16_t *tiled = nullptr, *lm_head_t = nullptr;
   std::mutex tiled_mu;
   std::atomic<bool> cancelled{false};
@@ -668,9 +669,9 @@ void begin_session(yuear_session &S, yuear_engine *E, int branches, int capacity
   S.history = S.alloc<int32_t>(size_t(S.history_cap) * sets);
   // prefill in chunks of up to 4096 tokens (~210 MB of scratch at the 3B
   // shape, plus the GEMMs' split-K partials): larger GEMMs fill the GPU
-  // better (M = 3000: 590 TFLOP/s against ~400 at M = 1024). A chunked
-  // prefill equals the one-pass prefill bit for bit when their GEMMs take the
-  // same tile shape and split count (shapes are chosen per M)
+  // better (whole 3B prefills: 3000 tokens at 920 TFLOP/s, 1024 at 730). A
+  // chunked prefill equals the one-pass prefill bit for bit when their GEMMs
+  // take the same tile shape and split count (chosen per M)
   S.chunk = std::min(capacity, 4096);
   const size_t T = S.chunk;
   S.px = S.alloc<uint16_t>(T * c.H);
@@ -1009,7 +1010,11 @@ void prefill(yuear_session &S, int b, const int32_t *ids, int n, uint16_t *logit
       HIPC(launch_qk_prep(qp, st));
       // The last layer's rows past K and V are read by the head alone, and only
       // the prompt's last one: its attention, projections and FFN run on that
-      // row, as in a decode step (301 tokens at 3072 wide: 88 us a prefill less).
+      // row with the GEMVs of one branch (301 tokens at 3072 wide: 88 us a prefill
+      // less). Their sums are in another order than the GEMMs', and a quantized
+      // engine's multiply the codes (s q + b, not rounded) where its GEMMs, and its
+      // steps of 3 and more branches, multiply the bf16 rows; a step of one or two
+      // branches does the same.
       const bool last = l + 1 == c.layers;
       if (last && start + T < n)
         break;
