@@ -218,134 +218,130 @@ __global__ __launch_bounds__(256) void qgemv_kernel(GemvParams p) {
 
   // 4. Row set blk, or with LOOP blk, blk + gridDim.x, ...: the next set's
   // loads are issued before this one's products, and no barrier separates the
-  // sets (a wave's sums pass through its own part of `res`).
-  static_assert(B * R * RW <= 64, "one lane per (row, branch) of a wave");
-  static_assert(R * RW % 2 == 0 || R * RW == 1, "a wave's rows are whole pairs, or one");
-  float *own = &res[0][0] + wave * (R * RW * B);  // [B][R * RW]
-  auto products = [&](int buf, int set) {
-    float acc[R][B];
+  // sets (a wave's sums pass through its own part of `res`). The products stand in
+  // the loop's body: as a function called for either buffer they took 3-23
+  // registers more a lane, often one wave a SIMD less (one pass, batch 2, 8 bits:
+  // 5120 x 4096 8.7 against 8.0 us, 5120 x 3072 6.7 against 6.2).
+  constexpr int ER = LOOP ? R * RW : ROWS;  // rows of an epilogue
+  static_assert(B * R * RW <= 64, "one thread per (row, branch)");
+  float *sums = &res[0][0] + (LOOP ? wave * (B * ER) : 0);  // [B][ER]
+  const int first = LOOP ? 0 : wave * (R * RW);
+  const int step = int(gridDim.x), sets = (p.n + ROWS - 1) / ROWS;
+  for (int set = blk; set < sets;) {  // (uniform)
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int b = 0; b < B; ++b)
-        acc[r][b] = 0.f;
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-      const int piece = li + q * L;
-      uint32_t xw[B][CPP * 4];
-      float sx[B];
-#pragma unroll
-      for (int b = 0; b < B; ++b) {
-#pragma unroll
-        for (int j = 0; j < CPP; ++j) {
-          const u32x4 v = xs[b][j * XS + piece];
-          xw[b][4 * j] = v.x;
-          xw[b][4 * j + 1] = v.y;
-          xw[b][4 * j + 2] = v.z;
-          xw[b][4 * j + 3] = v.w;
-        }
-        sx[b] = psum[b][piece];
+    for (int buf = 0; buf < (LOOP ? 2 : 1); ++buf, set += step) {
+      if constexpr (LOOP) {
+        if (set + step < sets)
+          load(1 - buf, set + step);
+        else if (set >= sets)
+          break;
       }
+      float acc[R][B];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const u32x4 w = wv[buf][r][q];
-        const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
-        uint32_t pr[4][4];
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int b = 0; b < B; ++b)
+          acc[r][b] = 0.f;
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-            pr[j][s] = ((wd[j] >> (4 * s)) & kPairMask) | kPairBias;
-        const float sc = bflo(sbv[buf][r][q]), bias = bfhi(sbv[buf][r][q]);
+      for (int q = 0; q < P; ++q) {
+        const int piece = li + q * L;
+        uint32_t xw[B][CPP * 4];
+        float sx[B];
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-          if constexpr (BITS == 4) {
-            float d0 = 0.f, d1 = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {  // word j <-> chunk j
-              d0 = dot2(pr[j][0], xw[b][4 * j], d0);
-              d1 = dot2(pr[j][1], xw[b][4 * j + 1], d1);
-              d0 = dot2(pr[j][2], xw[b][4 * j + 2], d0);
-              d1 = dot2(pr[j][3], xw[b][4 * j + 3], d1);
-            }
-            const float cb = __builtin_fmaf(-128.f, sc, bias);
-            acc[r][b] = __builtin_fmaf(sc, d0 + d1, __builtin_fmaf(cb, sx[b], acc[r][b]));
-          } else {
-            float lo = 0.f, hi = 0.f;
+          for (int j = 0; j < CPP; ++j) {
+            const u32x4 v = xs[b][j * XS + piece];
+            xw[b][4 * j] = v.x;
+            xw[b][4 * j + 1] = v.y;
+            xw[b][4 * j + 2] = v.z;
+            xw[b][4 * j + 3] = v.w;
+          }
+          sx[b] = psum[b][piece];
+        }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {  // word j: elements 4j..4j+3, pairs (0,2), (1,3)
-              const uint32_t x02 = xw[b][2 * j], x13 = xw[b][2 * j + 1];
-              lo = dot2(pr[j][0], x02, lo);
-              hi = dot2(pr[j][1], x02, hi);
-              lo = dot2(pr[j][2], x13, lo);
-              hi = dot2(pr[j][3], x13, hi);
+        for (int r = 0; r < R; ++r) {
+          const u32x4 w = wv[buf][r][q];
+          const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+          uint32_t pr[4][4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+              pr[j][s] = ((wd[j] >> (4 * s)) & kPairMask) | kPairBias;
+          const float sc = bflo(sbv[buf][r][q]), bias = bfhi(sbv[buf][r][q]);
+#pragma unroll
+          for (int b = 0; b < B; ++b) {
+            if constexpr (BITS == 4) {
+              float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {  // word j <-> chunk j
+                d0 = dot2(pr[j][0], xw[b][4 * j], d0);
+                d1 = dot2(pr[j][1], xw[b][4 * j + 1], d1);
+                d0 = dot2(pr[j][2], xw[b][4 * j + 2], d0);
+                d1 = dot2(pr[j][3], xw[b][4 * j + 3], d1);
+              }
+              const float cb = __builtin_fmaf(-128.f, sc, bias);
+              acc[r][b] = __builtin_fmaf(sc, d0 + d1, __builtin_fmaf(cb, sx[b], acc[r][b]));
+            } else {
+              float lo = 0.f, hi = 0.f;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {  // word j: elements 4j..4j+3, pairs (0,2), (1,3)
+                const uint32_t x02 = xw[b][2 * j], x13 = xw[b][2 * j + 1];
+                lo = dot2(pr[j][0], x02, lo);
+                hi = dot2(pr[j][1], x02, hi);
+                lo = dot2(pr[j][2], x13, lo);
+                hi = dot2(pr[j][3], x13, hi);
+              }
+              const float cb = __builtin_fmaf(-2176.f, sc, bias);
+              acc[r][b] = __builtin_fmaf(sc, __builtin_fmaf(16.f, hi, lo),
+                                         __builtin_fmaf(cb, sx[b], acc[r][b]));
             }
-            const float cb = __builtin_fmaf(-2176.f, sc, bias);
-            acc[r][b] = __builtin_fmaf(sc, __builtin_fmaf(16.f, hi, lo),
-                                       __builtin_fmaf(cb, sx[b], acc[r][b]));
           }
         }
       }
-    }
 
-    // 5. Row sums, then the epilogue of the wave's rows, one lane per (row or
-    // pair, branch).
-    __builtin_amdgcn_wave_barrier();  // the last set's sums have been read
+      // 5. Row sums, then the epilogue of the workgroup's rows (with LOOP of the
+      // wave's), one thread per (row or pair, branch).
+      if constexpr (LOOP)
+        __builtin_amdgcn_wave_barrier();  // the last set's sums have been read
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+      for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int b = 0; b < B; ++b) {
-        const float t = group_sum<L>(acc[r][b]);
-        if (li == 0)
-          own[b * (R * RW) + r * RW + sub] = t;
-      }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const int row0 = set * ROWS + wave * (R * RW);
-    if (p.epilogue == kEpiSwiGLU) {
-      if constexpr (R * RW % 2 == 0) {
-        const int b = lane / (R * RW / 2), i = lane % (R * RW / 2), row = row0 + 2 * i;
-        if (b < B && row + 1 < p.n) {
-          const float g = rbf(own[b * (R * RW) + 2 * i]), u = rbf(own[b * (R * RW) + 2 * i + 1]);
-          const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
-          p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
+        for (int b = 0; b < B; ++b) {
+          const float t = group_sum<L>(acc[r][b]);
+          if (li == 0)
+            sums[b * ER + first + r * RW + sub] = t;
         }
-      } else if constexpr (!LOOP) {  // one row a wave: a pair's rows are in two waves
+      if constexpr (LOOP) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      } else {
         __syncthreads();
-        const float *gate = &res[0][0] + (tid & 1) * (2 * B), *up = gate + B;  // [wave][B]
-        const int b = tid >> 1, row = set * ROWS + 2 * (tid & 1);
-        if (b < B && row + 1 < p.n) {
-          const float g = rbf(gate[b]), u = rbf(up[b]);
-          const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
-          p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
+      }
+      const int row0 = set * ROWS + (LOOP ? wave * ER : 0), et = LOOP ? lane : tid;
+      if (p.epilogue == kEpiSwiGLU) {
+        if constexpr (ER % 2 == 0) {  // (a pair's rows are in one epilogue)
+          const int b = et / (ER / 2), i = et % (ER / 2), row = row0 + 2 * i;
+          if (b < B && row + 1 < p.n) {
+            const float g = rbf(sums[b * ER + 2 * i]), u = rbf(sums[b * ER + 2 * i + 1]);
+            const float act = rbf(g * (1.0f / (1.0f + expf(-g))));
+            p.y[size_t(b) * p.y_stride + (row >> 1)] = f2bf(act * u);
+          }
+        }
+      } else {
+        const int b = et / ER, i = et % ER, row = row0 + i;
+        if (b < B && row < p.n) {
+          uint16_t *y = p.y + size_t(b) * p.y_stride + row;
+          float v = sums[b * ER + i];
+          if (p.epilogue == kEpiResidual)
+            v = bf2f(*y) + rbf(v);
+          *y = f2bf(v);
         }
       }
-    } else {
-      const int b = lane / (R * RW), i = lane % (R * RW), row = row0 + i;
-      if (b < B && row < p.n) {
-        uint16_t *y = p.y + size_t(b) * p.y_stride + row;
-        float v = own[b * (R * RW) + i];
-        if (p.epilogue == kEpiResidual)
-          v = bf2f(*y) + rbf(v);
-        *y = f2bf(v);
-      }
     }
-  };
-  if constexpr (!LOOP) {
-    products(0, blk);
-  } else {
-    const int step = int(gridDim.x), sets = (p.n + ROWS - 1) / ROWS;
-    for (int set = blk; set < sets; set += 2 * step) {
-      const bool more = set + step < sets;  // uniform
-      if (more)
-        load(1, set + step);
-      products(0, set);
-      if (!more)
-        break;
-      if (set + 2 * step < sets)
-        load(0, set + 2 * step);
-      products(1, set + step);
-    }
+    if constexpr (!LOOP)
+      break;
   }
   if (p.advance && blk == 0 && tid < p.batch)
     p.advance[tid] += 1;
@@ -386,10 +382,10 @@ hipError_t launch_r(const GemvParams &p, hipStream_t s, int grid) {
 // 32769 x 2048 9.6 against 9.9 us looped). Measured on MI355X, us, cold
 // weights, before (one pass, at least 1024 workgroups) -> now, batch 1 / 2:
 //   4 bits: 5120 x 3072  5.1 -> 4.6 / 7.6 -> 6.0;  16384 x 3072 SwiGLU
-//   8.4 -> 8.5 / 12.6 -> 10.2;  83968 x 3072  26.8 -> 26.3 / 41.0 -> 32.2;
-//   12288 x 2048 SwiGLU  5.9 -> 5.5 / 8.3 -> 7.0
-//   8 bits: 6.8 -> 6.0 / 9.5 -> 7.6;  13.2 -> 12.8 / 16.7 -> 16.0;
-//   47.6 -> 46.4 / 65.2 -> 57.4;  7.8 -> 7.7 / 10.6 -> 9.6
+//   8.4 -> 8.5 / 12.6 -> 10.1;  83968 x 3072  26.7 -> 25.9 / 41.3 -> 31.7;
+//   12288 x 2048 SwiGLU  5.8 -> 5.2 / 8.2 -> 6.8
+//   8 bits: 6.7 -> 5.8 / 9.3 -> 7.5;  12.4 -> 12.7 / 16.8 -> 16.1;
+//   47.6 -> 47.1 / 64.6 -> 57.4;  7.7 -> 7.5 / 10.3 -> 9.5
 // Without a norm the staging is cheap and more workgroups win (3072 x 8192 at
 // 8 bits, batch 2: 10.3 in one pass, 12.2 in the loop).
 template <int B, int BITS, int L, int P>
@@ -408,7 +404,7 @@ hipError_t launch_lp(const GemvParams &p, hipStream_t s) {
         if (sets(2) >= 512)
           return launch_r<B, BITS, L, P, 2, false>(p, s, sets(2));
       }
-      // (SwiGLU needs a pair's rows in one wave, or the barrier of the one-pass form)
+      // (SwiGLU needs a pair's rows in one epilogue)
       if (sets(1) > 512 && (L < 64 || p.epilogue != kEpiSwiGLU))
         return launch_r<B, BITS, L, P, 1, true>(p, s, 512);
     }
